@@ -454,10 +454,11 @@ void rlcd_objective(laya_ctx* ctx, const float* logits, const float* targets, co
                     int n_items, int total_options, int max_options, int groups, const double* draws, double sigma,
                     double spherical, double rps, double ce_weight, double scale, float* grad, double* losses);
 // DecisionModel.ReadOut (DecisionModel.cs:170-226) per item: probs [n_items][na], features [n_items][4]
-// (may be null); states are the head output rows, opt_off [n_items + 1] the items' option offsets.
+// (may be null); hidden [n_items][a1] is scratch; states are the head output rows, opt_off [n_items + 1] the
+// items' option offsets.
 void decision_readout(laya_ctx* ctx, const float* scores, const int* opt_off, const int* seg_start, int n_items,
                       const float* states, int d, const float* w1, const float* b1, int a1, const float* w2,
-                      const float* b2, int na, float* probs, float* features);
+                      const float* b2, int na, float* hidden, float* probs, float* features);
 // rows: the number of rows of qkv / context / dcontext (the dO·O row constants span all of them); amax
 // (optional): max|dqkv| folded into a magnitude word group.
 void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float* context, const float* lse,

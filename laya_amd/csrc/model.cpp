@@ -1497,9 +1497,9 @@ int laya_model_readout(laya_model* m, float* logits_host, float* act_probs_host,
         const int a1 = m->find("act_head.0.bias"), na_i = m->find("act_head.2.bias");
         const int w1 = m->find("act_head.0.weight"), w2 = m->find("act_head.2.weight");
         const int A1 = (int)m->params[a1].numel, NA = (int)m->params[na_i].numel, n = m->nseg;
-        float* out = static_cast<float*>(m->ctx->workspace(8, sizeof(float) * (size_t)std::max(1, n) * (NA + 4)));
+        float* out = static_cast<float*>(m->ctx->workspace(8, sizeof(float) * (size_t)std::max(1, n) * (NA + 4 + A1)));
         decision_readout(m->ctx, m->scores, m->cur.opt_off, m->cur.seg_start, n, m->head_out, m->d(), m->W(w1),
-                         m->W(a1), A1, m->W(w2), m->W(na_i), NA, out, out + (size_t)n * NA);
+                         m->W(a1), A1, m->W(w2), m->W(na_i), NA, out + (size_t)n * (NA + 4), out, out + (size_t)n * NA);
         LAYA_HIP(hipMemcpyAsync(act_probs_host, out, sizeof(float) * (size_t)n * NA, hipMemcpyDeviceToHost,
                                 m->ctx->stream));
         if (features_host)
