@@ -1363,15 +1363,31 @@ __global__ __launch_bounds__(WT_THREADS, 1) void gemm_x6w_kernel(GemmParams p) {
 // fp32, though possibly NaN where fp32 gives an infinity).
 constexpr int AMAX_BLOCKS = 1024, AMAX_SLOTS = 6;
 
-__global__ __launch_bounds__(256) void absmax_kernel(const float* __restrict__ x, int rows, int cols, long ld,
-                                                     int vec, unsigned* out) {
+constexpr int AMAX_OPERANDS = 3;
+struct AmaxJob {
+    const float* x;
+    int rows, cols;
+    long ld;
+    int vec, blocks;
+    unsigned* out;
+};
+struct AmaxJobs {
+    AmaxJob job[AMAX_OPERANDS];
+};
+
+// Up to three operands in one launch, each over its own run of blocks: a product's operands are measured together,
+// because a short launch costs its latency whatever it reads (3.6 us for 1.5 to 7 MB).
+__global__ __launch_bounds__(256) void absmax_kernel(AmaxJobs jobs) {
+    int bid = blockIdx.x, j = 0;
+    while (j + 1 < AMAX_OPERANDS && bid >= jobs.job[j].blocks) bid -= jobs.job[j++].blocks;
+    const AmaxJob q = jobs.job[j];
     unsigned m = 0;
     const int tid = threadIdx.x;
-    if (vec && ld == cols) {
-        const long n4 = (long)rows * cols / 4;
-        const f32x4* x4 = reinterpret_cast<const f32x4*>(x);
-        const long stride = (long)gridDim.x * 256;
-        long i = (long)blockIdx.x * 256 + tid;
+    if (q.vec && q.ld == q.cols) {
+        const long n4 = (long)q.rows * q.cols / 4;
+        const f32x4* x4 = reinterpret_cast<const f32x4*>(q.x);
+        const long stride = (long)q.blocks * 256;
+        long i = (long)bid * 256 + tid;
         for (; i + 3 * stride < n4; i += 4 * stride) {
             f32x4 v[4];
 #pragma unroll
@@ -1380,16 +1396,16 @@ __global__ __launch_bounds__(256) void absmax_kernel(const float* __restrict__ x
             for (int u = 0; u < 4; ++u) m = max(m, amax_bits4(v[u]));
         }
         for (; i < n4; i += stride) m = max(m, amax_bits4(x4[i]));
-    } else if (vec) {
-        for (int r = blockIdx.x; r < rows; r += gridDim.x) {
-            const f32x4* row = reinterpret_cast<const f32x4*>(x + (long)r * ld);
-            for (int c = tid; c < cols / 4; c += 256) m = max(m, amax_bits4(row[c]));
+    } else if (q.vec) {
+        for (int r = bid; r < q.rows; r += q.blocks) {
+            const f32x4* row = reinterpret_cast<const f32x4*>(q.x + (long)r * q.ld);
+            for (int c = tid; c < q.cols / 4; c += 256) m = max(m, amax_bits4(row[c]));
         }
     } else {
-        for (int r = blockIdx.x; r < rows; r += gridDim.x)
-            for (int c = tid; c < cols; c += 256) m = max(m, amax_bits(x[(long)r * ld + c]));
+        for (int r = bid; r < q.rows; r += q.blocks)
+            for (int c = tid; c < q.cols; c += 256) m = max(m, amax_bits(q.x[(long)r * q.ld + c]));
     }
-    block_amax_fold(m, out);
+    block_amax_fold(m, q.out);
 }
 
 // ------------------------------------------------------------- split products on 192 x 256 tiles
@@ -2577,46 +2593,80 @@ void absmax_multi(laya_ctx* ctx, const float* arena, const long* off, const int*
     check_launch("absmax_multi_kernel");
 }
 
-// max|x| of a rows x cols operand folded into *out (0 beforehand for the operand's own maximum).
-void absmax_into(laya_ctx* ctx, const float* x, int rows, int cols, long ld, unsigned* out) {
+namespace {
+
+AmaxJob amax_job(const float* x, int rows, int cols, long ld, unsigned* out) {
     const long n = (long)rows * cols;
-    if (n <= 0) return;
-    ProfileScope scope(ctx, "absmax", 0.0, 4.0 * n);
     const int vec = cols % 4 == 0 && ld % 4 == 0 && aligned16(x);
     const long per_block = 256L * 4 * 8;  // eight float4 per thread
     const int blocks = (int)std::max(1L, std::min<long>(AMAX_BLOCKS, (n + per_block - 1) / per_block));
-    LAYA_LAUNCH(absmax_kernel, dim3(vec && ld == cols ? blocks : std::min(blocks, std::max(rows, 1))),
-                       dim3(256), 0, ctx->stream, x, rows, cols, ld, vec, out);
+    return AmaxJob{x, rows, cols, ld, vec, vec && ld == cols ? blocks : std::min(blocks, std::max(rows, 1)), out};
+}
+
+void launch_absmax(laya_ctx* ctx, const AmaxJob* job, int n) {
+    AmaxJobs jobs{};
+    int blocks = 0;
+    double elements = 0.0;
+    for (int i = 0; i < n; ++i) {
+        if (job[i].rows <= 0 || job[i].cols <= 0) continue;
+        elements += (double)job[i].rows * job[i].cols;
+        for (AmaxJob& j : jobs.job)
+            if (!j.blocks) {
+                j = job[i];
+                break;
+            }
+        blocks += job[i].blocks;
+    }
+    if (!blocks) return;
+    ProfileScope scope(ctx, "absmax", 0.0, 4.0 * elements);
+    LAYA_LAUNCH(absmax_kernel, dim3(blocks), dim3(256), 0, ctx->stream, jobs);
     check_launch("absmax_kernel");
+}
+
+// An operand of a product and where its magnitude word group goes.
+struct Operand {
+    AmaxRef ref;
+    const float* x;
+    int rows, cols;
+    long ld;
+    const unsigned** word;
+};
+
+// The magnitude words of a product's operands: the caller's where it keeps them (measured now if not known yet: an
+// unknown word holds zero), else the context's next groups; everything there is to measure in one launch.
+void operand_amaxes(laya_ctx* ctx, std::initializer_list<Operand> operands) {
+    AmaxJob job[AMAX_OPERANDS];
+    int n = 0;
+    for (const Operand& o : operands) {
+        if (!o.ref.word) {
+            unsigned* w = operand_ring_word(ctx);
+            *o.word = w;
+            job[n++] = amax_job(o.x, o.rows, o.cols, o.ld, w);
+        } else {
+            *o.word = o.ref.word;
+            if (!*o.ref.known) {
+                job[n++] = amax_job(o.x, o.rows, o.cols, o.ld, o.ref.word);
+                *o.ref.known = 1;
+            }
+        }
+    }
+    if (n) launch_absmax(ctx, job, n);
+}
+
+}  // namespace
+
+// max|x| of a rows x cols operand folded into *out (0 beforehand for the operand's own maximum).
+void absmax_into(laya_ctx* ctx, const float* x, int rows, int cols, long ld, unsigned* out) {
+    const AmaxJob job = amax_job(x, rows, cols, ld, out);
+    launch_absmax(ctx, &job, 1);
 }
 
 namespace {
 
-// max|x| of a rows x cols operand into the context's next word group; returns it. `slot` names the operand's
-// role for the callers' bookkeeping only.
-const unsigned* operand_absmax(laya_ctx* ctx, int slot, const float* x, int rows, int cols, long ld) {
-    (void)slot;
-    unsigned* out = operand_ring_word(ctx);
-    absmax_into(ctx, x, rows, cols, ld, out);
-    return out;
-}
-
-// The magnitude word of an operand: the caller's (measured now if it is not known yet: an unknown word
-// holds zero) or the context's slot `slot`, measured now.
-const unsigned* operand_amax(laya_ctx* ctx, AmaxRef r, int slot, const float* x, int rows, int cols, long ld) {
-    if (!r.word) return operand_absmax(ctx, slot, x, rows, cols, ld);
-    if (!*r.known) {
-        absmax_into(ctx, x, rows, cols, ld, r.word);
-        *r.known = 1;
-    }
-    return r.word;
-}
-
 // An NT product on 256-wide tiles (wide or tall) as two-piece fp16 products: both operands' magnitudes
 // are taken first (outside the product's profile scope) and the launchers below see amax_a set.
 void prepare_pair_nt(laya_ctx* ctx, GemmParams& p, AmaxRef ra, AmaxRef rb) {
-    p.amax_a = operand_amax(ctx, ra, 0, p.A, p.M, p.K, p.lda);
-    p.amax_b = operand_amax(ctx, rb, 1, p.B, p.N, p.K, p.ldb);
+    operand_amaxes(ctx, {{ra, p.A, p.M, p.K, p.lda, &p.amax_a}, {rb, p.B, p.N, p.K, p.ldb, &p.amax_b}});
     p.b_one = rb.bf16 ? 1 : 0;
 }
 
@@ -2942,7 +2992,9 @@ unsigned* operand_ring_word(laya_ctx* ctx) {
 
 const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, int slot, const float* x, int rows, int cols, long ld) {
     LAYA_REQUIRE(slot >= 0 && slot < AMAX_SLOTS, "operand_amax_ref: no such slot");
-    return operand_amax(ctx, r, slot, x, rows, cols, ld);
+    const unsigned* word = nullptr;
+    operand_amaxes(ctx, {{r, x, rows, cols, ld, &word}});
+    return word;
 }
 
 void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K, const float* A, long lda,
@@ -2986,11 +3038,9 @@ void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K
         (ctx->matmul_split & cls) && gemm_fits_h(p, layout == GemmLayout::NN, false) &&
         (layout == GemmLayout::TN ? ep == GemmEpilogue::Accumulate
                                   : operand_fast(p.A, p.lda, p.vec_a, true, p.M, p.K))) {
-        if (layout == GemmLayout::NN)
-            p.amax_a = operand_amax(ctx, amax_a, 0, p.A, p.M, p.K, p.lda);
-        else
-            p.amax_a = operand_amax(ctx, amax_a, 0, p.A, p.K, p.M, p.lda);
-        p.amax_b = operand_amax(ctx, amax_b, 1, p.B, p.K, p.N, p.ldb);
+        const bool nn = layout == GemmLayout::NN;
+        operand_amaxes(ctx, {{amax_a, p.A, nn ? p.M : p.K, nn ? p.K : p.M, p.lda, &p.amax_a},
+                             {amax_b, p.B, p.K, p.N, p.ldb, &p.amax_b}});
     }
     // C's magnitude: folded in by a two-piece kernel's epilogue, else measured after the product.
     bool measure = amax_c && !p.amax_c;
@@ -3225,9 +3275,10 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
     s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * WT * WT));
     const bool pair = !half && (ctx->matmul_pair & 6) == 6;
     if (pair) {
-        nn.amax_a = tn.amax_a = operand_amax(ctx, amax_dy, 0, nn.A, rows, out, nn.lda);
-        nn.amax_b = operand_amax(ctx, amax_W, 1, nn.B, out, in, nn.ldb);
-        tn.amax_b = operand_amax(ctx, amax_x, 2, tn.B, rows, in, tn.ldb);
+        operand_amaxes(ctx, {{amax_dy, nn.A, rows, out, nn.lda, &nn.amax_a},
+                             {amax_W, nn.B, out, in, nn.ldb, &nn.amax_b},
+                             {amax_x, tn.B, rows, in, tn.ldb, &tn.amax_b}});
+        tn.amax_a = nn.amax_a;
         nn.amax_c = nn.R ? nullptr : amax_dx;
         *folded = nn.amax_c != nullptr;
     }
