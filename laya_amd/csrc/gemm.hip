@@ -25,6 +25,7 @@
 // fifth slower on short-K products.
 #include "common.hpp"
 #include "elementwise.hpp"
+#include "gemm_short.hpp"
 #include "split.hpp"
 
 namespace laya {
@@ -2926,6 +2927,24 @@ GemmParams make_params(int M, int N, int K, const float* A, long lda, const floa
     return p;
 }
 
+ShortGemm short_params(int M, int N, int K, const float* A, long lda, const float* B, long ldb, float* C, long ldc,
+                       const float* bias, const float* R, long ldr) {
+    ShortGemm g{};
+    g.A = A;
+    g.B = B;
+    g.C = C;
+    g.bias = bias;
+    g.R = R;
+    g.lda = lda;
+    g.ldb = ldb;
+    g.ldc = ldc;
+    g.ldr = ldr;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    return g;
+}
+
 // Splits K into `splits` slices of a multiple of BK; returns the realised split count.
 int set_splits(GemmParams& p, int splits) {
     int kps = (p.K + splits - 1) / splits;
@@ -3001,6 +3020,16 @@ void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K
           const float* B, long ldb, float* C, long ldc, const float* bias, const float* R, long ldr,
           const __bf16* A16, const __bf16* B16, AmaxRef amax_a, AmaxRef amax_b, unsigned* amax_c) {
     if (M == 0 || N == 0) return;
+    if (layout == GemmLayout::TN ? ep == GemmEpilogue::Accumulate && !bias && !R : ep == GemmEpilogue::Store) {
+        ShortGemm g = short_params(M, N, K, A, lda, B, ldb, C, ldc, bias, R, ldr);
+        g.amax = amax_c;
+        const ShortEpilogue se =
+            ep == GemmEpilogue::Store ? ShortEpilogue::Store : ShortEpilogue::Accumulate;
+        if (short_gemm_pays(ctx, layout, se, g)) {
+            short_gemm(ctx, layout, se, g);
+            return;
+        }
+    }
     GemmParams p = make_params(M, N, K, A, lda, B, ldb, C, ldc, bias, R, ldr);
     p.A16 = A16;
     p.B16 = B16;
@@ -3081,6 +3110,16 @@ void gemm_rope(laya_ctx* ctx, int M, int N, int K, const float* A, const float* 
                const int* pos, const float* cos_t, const float* sin_t, int rope_cols, const __bf16* A16,
                const __bf16* B16, AmaxRef amax_a, AmaxRef amax_b, unsigned* amax_c) {
     if (M == 0 || N == 0) return;
+    ShortGemm g = short_params(M, N, K, A, K, B, K, C, N, bias, nullptr, 0);
+    g.amax = amax_c;
+    g.rope_pos = pos;
+    g.rope_cos = cos_t;
+    g.rope_sin = sin_t;
+    g.rope_cols = rope_cols;
+    if (rope_cols <= N && pos && cos_t && sin_t && short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Rope, g)) {
+        short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Rope, g);
+        return;
+    }
     GemmParams p = make_params(M, N, K, A, K, B, K, C, N, bias, nullptr, 0);
     [&] {
         p.A16 = A16;
@@ -3171,6 +3210,15 @@ void gemm_geglu(laya_ctx* ctx, int M, int inter, int K, const float* x, const fl
                 unsigned* amax_act) {
     if (M == 0) return;
     const int N = 2 * inter;
+    ShortGemm g = short_params(M, N, K, x, K, W, K, wide, N, bias, nullptr, 0);
+    g.amax = amax_act;
+    g.act = act;
+    g.act16 = act16;
+    g.inter = inter;
+    if (short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g)) {
+        short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g);
+        return;
+    }
     GemmParams p = make_params(M, N, K, x, K, W, K, wide, N, bias, nullptr, 0);
     p.A16 = x16;
     p.B16 = W16;
@@ -3338,6 +3386,16 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
                              const __bf16* x16, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx,
                              bool* folded) {
     if (rows == 0) return;
+    {
+        ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
+        const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
+        nn.amax = amax_dx;
+        if (short_pair_pays(ctx, nn, tn)) {
+            short_gemm_pair(ctx, nn, tn);
+            *folded = amax_dx != nullptr;
+            return;
+        }
+    }
     // dx[rows, in] = dy[rows, out] · W[out, in]       (NN, K = out)
     GemmParams nn = make_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
     nn.mode = STORE;

@@ -38,3 +38,64 @@ def test_readout_option_counts(ctx):
     np.testing.assert_allclose(feats, feats_o, atol=1e-5)
     np.testing.assert_allclose(probs, probs_o, atol=1e-5)
     m.close()
+
+
+def _bf16(a):
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32).astype(np.uint64)
+    return (((u + 0x7fff + ((u >> 16) & 1)) >> 16) << 16).astype(np.uint32).view(np.float32)
+
+
+def _rel(a, b):
+    return np.linalg.norm(np.asarray(a, np.float64) - b) / max(np.linalg.norm(b), 1e-300)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("rows,fan_in,fan_out", [
+    (1, 32, 4), (5, 64, 64), (31, 96, 100), (33, 128, 132), (63, 256, 256), (65, 800, 96), (129, 768, 2304),
+    (404, 1024, 544), (700, 768, 768), (512, 2048, 1024), (1100, 1024, 5248), (100, 100, 36), (97, 66, 30)])
+def test_short_products(ctx, precision, rows, fan_in, fan_out):
+    """Linear layers over few rows, forward (with bias and residual) and backward, at the edges of the 32- and 64-wide
+    tiles and of the 32-deep stages, on both sides of the rules that choose among them, and shapes that they refuse (a K
+    that is no multiple of 32, widths that are no multiple of 4); against fp64 on the same operands (rounded to bf16
+    first for bf16 products). Operand rows spread over four decades and start from an unaligned size. fp32 accumulation
+    rounds to about 2^-24 per addition: 1e-6 relative L2, as the other products' tests hold."""
+    from laya_amd import ops
+    from laya_amd.device import Context, DeviceArray
+    c = ctx if precision == "fp32" else Context(0)
+    c.set_matmul_precision(precision)
+    r = np.random.default_rng(rows * 7 + fan_out)
+    x = (r.standard_normal((rows, fan_in)) * 10.0 ** r.uniform(-2, 2, (rows, 1))).astype(np.float32)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    b = r.standard_normal(fan_out).astype(np.float32)
+    res = r.standard_normal((rows, fan_out)).astype(np.float32)
+    dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
+    dW0 = (1e-3 * r.standard_normal(W.shape)).astype(np.float32)
+    low = (lambda a: _bf16(a).astype(np.float64)) if precision == "bf16" else (lambda a: a.astype(np.float64))
+    Wp, bp = ops.Parameter(c, "W", W), ops.Parameter(c, "b", b)
+    xd, yd = DeviceArray.from_numpy(c, x), DeviceArray(c, (rows, fan_out))
+    ops.linear(Wp, bp, xd, rows, yd, residual=DeviceArray.from_numpy(c, res))
+    assert _rel(yd.numpy(), low(x) @ low(W).T + b + res) < 1e-6
+    Wp.gradient_buffer().upload(dW0)
+    dxd = DeviceArray(c, (rows, fan_in))
+    ops.linear_backward(Wp, bp, xd, DeviceArray.from_numpy(c, dy), rows, dxd)
+    assert _rel(dxd.numpy(), low(dy) @ low(W)) < 1e-6
+    assert _rel(Wp.gradient_buffer().numpy(), dW0 + low(dy).T @ low(x)) < 1e-6
+    if c is not ctx:
+        c.close()
+
+
+def test_short_product_with_non_finite_operands(ctx):
+    """A NaN or infinity stays in its own row: the scale comes from the finite values (the rows beside it are held to
+    fp64 as above)."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    r = np.random.default_rng(3)
+    x = r.standard_normal((96, 256)).astype(np.float32)
+    W = (0.02 * r.standard_normal((128, 256))).astype(np.float32)
+    x[40, 17], x[7, 200] = np.inf, np.nan
+    yd = DeviceArray(ctx, (96, 128))
+    ops.linear(ops.Parameter(ctx, "W", W), None, DeviceArray.from_numpy(ctx, x), 96, yd)
+    y = yd.numpy()
+    bad = np.isin(np.arange(96), (7, 40))
+    assert not np.isfinite(y[bad]).any()
+    assert _rel(y[~bad], x[~bad].astype(np.float64) @ W.astype(np.float64).T) < 1e-6
