@@ -66,13 +66,17 @@ struct Params {
 struct BlockCoord {
     int seg, head, row0;
 };
+// ROWS: the workgroup's rows, BLOCK_ROWS or a part of them (BLOCK_ROWS / ROWS consecutive workgroups per entry and head).
+template <int ROWS = BLOCK_ROWS>
 __device__ __forceinline__ BlockCoord block_coord(const Params& p) {
     if (p.blocks) {
-        const unsigned i = blockIdx.x / (unsigned)p.heads;
+        constexpr unsigned PARTS = BLOCK_ROWS / ROWS;
+        const unsigned at = blockIdx.x / PARTS, i = at / (unsigned)p.heads;
         const unsigned e = (unsigned)p.blocks[i];
-        return {(int)(e >> 16), (int)(blockIdx.x - i * (unsigned)p.heads), (int)(e & 0xffffu) * BLOCK_ROWS};
+        return {(int)(e >> 16), (int)(at - i * (unsigned)p.heads),
+                (int)(e & 0xffffu) * BLOCK_ROWS + (int)(blockIdx.x % PARTS) * ROWS};
     }
-    return {(int)blockIdx.y, (int)blockIdx.z, (int)blockIdx.x * BLOCK_ROWS};
+    return {(int)blockIdx.y, (int)blockIdx.z, (int)blockIdx.x * ROWS};
 }
 
 template <int D> struct Shape {
@@ -552,19 +556,58 @@ __device__ __forceinline__ void swz_col_frag(const __bf16* planes, int r0, int d
 }
 
 // NP = 3: three-piece bf16 split products; NP = 2: two-piece fp16 products of scaled operands.
-template <int D, bool DROP, int NP = 3>
-__global__ __launch_bounds__(THREADS, 2) void attn_fwd_x6_kernel(Params p) {
+// Short attention: workgroups of 32 rows whose four waves take a 32-row subtile of the streamed operand each, for grids
+// that would leave most of the chip idle with 128 rows to a workgroup. The waves' accumulators are summed through LDS.
+constexpr int CUT_TILE = 4 * WAVE_ROWS;
+
+__device__ __forceinline__ void park(float* red, int wave, int lane, const f32x16 (&acc)[2], float scale) {
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[(wave * 32 + dt * 16 + r) * 64 + lane] = acc[dt][r] * scale;
+}
+// Registers 4g … 4g + 3 of tile dt that wave v parked: d = 32·dt + 8g + 4h ….
+__device__ __forceinline__ f32x4 parked(const float* red, int v, int lane, int dt, int g) {
+    const float* x = red + (v * 32 + dt * 16 + 4 * g) * 64 + lane;
+    return f32x4{x[0], x[64], x[128], x[192]};
+}
+// Wave g's d = 8g … 8g + 7 of both halves summed over the waves in order, rotated back when asked, written to dst.
+__device__ __forceinline__ unsigned store_parked(const float* red, int lane, int g, const Params& p, bool rope, int t,
+                                                 float* dst) {
+    const int i0 = 8 * g + 4 * (lane >> 5);
+    f32x4 a = parked(red, 0, lane, 0, g), b = parked(red, 0, lane, 1, g);
+#pragma unroll
+    for (int v = 1; v < 4; ++v) {
+        a += parked(red, v, lane, 0, g);
+        b += parked(red, v, lane, 1, g);
+    }
+    if (rope) {
+        const f32x4 c = ld4(p.cos_t + (long)t * 32 + i0), s = ld4(p.sin_t + (long)t * 32 + i0);
+        const f32x4 x = a * c + b * s;
+        b = b * c - a * s;
+        a = x;
+    }
+    st4(dst + i0, a);
+    st4(dst + 32 + i0, b);
+    return max(amax_bits4(a), amax_bits4(b));
+}
+
+template <int D, bool DROP, int NP = 3, int ROWS = BLOCK_ROWS>
+__global__ __launch_bounds__(THREADS, ROWS == BLOCK_ROWS ? 2 : 1) void attn_fwd_x6_kernel(Params p) {
     static_assert(D == 64, "split-product attention is written for head_dim 64");
+    constexpr bool CUT = ROWS == WAVE_ROWS;  // few rows: the waves share their queries and take a subtile each
+    static_assert(!CUT || NP == 2, "the shared form is written for two-piece products");
+    constexpr int TILE = CUT ? CUT_TILE : laya::TILE;
     __shared__ __attribute__((aligned(16))) __bf16 Ks[NP * TILE * 64];  // K tile, swizzled [key][d]
     __shared__ __attribute__((aligned(16))) __bf16 Vs[NP * TILE * 64];  // V tile, swizzled [key][d]
 
-    const BlockCoord bc = block_coord(p);
+    const BlockCoord bc = block_coord<ROWS>(p);
     const int seg = bc.seg, head = bc.head;
     const int start = p.seg_start[seg], L = p.seg_len[seg];
     const int qb0 = bc.row0;
     if (qb0 >= L) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, lr = lane & 31;
-    const int q0w = qb0 + wave * WAVE_ROWS;
+    const int q0w = CUT ? qb0 : qb0 + wave * WAVE_ROWS;
     const int q = q0w + lr;
     const bool qvalid = q < L;
     const int hw = p.half_window;
@@ -595,7 +638,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_x6_kernel(Params p) {
     int wbeg = 0, wend = L;
     if (hw >= 0) {
         kbeg = max(0, qb0 - hw);
-        kend = min(L, qb0 + BLOCK_ROWS + hw);
+        kend = min(L, qb0 + ROWS + hw);
         wbeg = max(0, q0w - hw);
         wend = min(L, q0w + WAVE_ROWS + hw);
     }
@@ -624,7 +667,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_x6_kernel(Params p) {
             fetch_rows<TILE>(vst, vbase, stride, L, kt0 + TILE);
         }
 #pragma unroll
-        for (int st = 0; st < TILE / 32; ++st) {
+        for (int st = CUT ? wave : 0; st < (CUT ? wave + 1 : TILE / 32); ++st) {
             const int kbs = kt0 + 32 * st;
             // Wave-uniform: outside this wave's window, or a wave whose rows all lie past the segment end.
             if (kbs >= wend || kbs + 32 <= wbeg || kbs >= kend || q0w >= L) continue;
@@ -705,6 +748,44 @@ __global__ __launch_bounds__(THREADS, 2) void attn_fwd_x6_kernel(Params p) {
 
     const float lt = l + __shfl_xor(l, 32, 64);
     unsigned am = 0;
+    if constexpr (CUT) {
+        // The waves' sums brought to the largest of their units 2^(m − ep); wave w writes d = 8w … 8w + 7 of both halves.
+        __shared__ float unit_s[4][32], l_s[4][32];
+        float* red = reinterpret_cast<float*>(Ks);  // [wave][accumulator register][lane]
+        __syncthreads();
+        park(red, wave, lane, o, 1.0f);
+        if (h == 0) {
+            unit_s[wave][lr] = lt > 0.0f ? m - (float)ep : NEG_INF;
+            l_s[wave][lr] = lt;
+        }
+        __syncthreads();
+        float top = NEG_INF, f[4], sum = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) top = fmaxf(top, unit_s[v][lr]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            f[v] = top > NEG_INF ? fast_exp2(unit_s[v][lr] - top) : 0.0f;
+            sum += f[v] * l_s[v][lr];
+        }
+        const float inv = sum > 0.0f ? ldexpf(1.0f / sum, -eq) : 0.0f;
+        if (qvalid) {
+            const long at = (long)(start + q) * p.hidden + qcol + 8 * wave + 4 * h;
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) {
+                f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x += f[v] * parked(red, v, lane, dt, wave);
+                x *= inv;
+                st4(p.context + at + 32 * dt, x);
+                if (p.context16) *reinterpret_cast<bf16x4*>(p.context16 + at + 32 * dt) = __builtin_convertvector(x, bf16x4);
+                am = max(am, amax_bits4(x));
+            }
+            if (wave == 0 && h == 0)
+                p.lse[(long)(start + q) * p.heads + head] = sum > 0.0f ? top + log2f(sum) : __builtin_huge_valf();
+        }
+        block_amax_fold(am, p.amax);
+        return;
+    }
     if (qvalid) {
         const float inv = lt > 0.0f ? (NP == 2 ? ldexpf(1.0f / lt, -eq) : 1.0f / lt) : 0.0f;
         am = store_acc<D>(o, p.context + (long)(start + q) * p.hidden + qcol, h, inv);
@@ -981,22 +1062,25 @@ constexpr int BT = 32;
 // Each wave owns 32 keys: K split once into registers, V split once into the block's LDS planes. The
 // query tiles are committed to one swizzled layout each (Q and dO), the next tile's rows load while the
 // current one is multiplied, and the products over queries read Qᵀ and dOᵀ with the transposing reads.
-template <int D, bool DROP, int NP = 3>
-__global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
+template <int D, bool DROP, int NP = 3, int ROWS = BLOCK_ROWS>
+__global__ __launch_bounds__(THREADS, ROWS == BLOCK_ROWS ? 2 : 1) void attn_bwd_dkv_x6_kernel(Params p) {
     static_assert(D == 64, "split-product attention is written for head_dim 64");
+    constexpr bool CUT = ROWS == WAVE_ROWS;  // few rows: the waves share their keys and take a query subtile each
+    static_assert(!CUT || NP == 2, "the shared form is written for two-piece products");
+    constexpr int BT = CUT ? CUT_TILE : laya::BT;
     __shared__ __attribute__((aligned(16))) __bf16 Qs[NP * BT * 64];
     __shared__ __attribute__((aligned(16))) __bf16 Os[NP * BT * 64];
-    __shared__ __attribute__((aligned(16))) __bf16 Vs[NP * BLOCK_ROWS * 64];
+    __shared__ __attribute__((aligned(16))) __bf16 Vs[NP * ROWS * 64];
     __shared__ __attribute__((aligned(16))) float lse_s[BT];
     __shared__ __attribute__((aligned(16))) float dot_s[BT];
 
-    const BlockCoord bc = block_coord(p);
+    const BlockCoord bc = block_coord<ROWS>(p);
     const int seg = bc.seg, head = bc.head;
     const int start = p.seg_start[seg], L = p.seg_len[seg];
     const int kb0 = bc.row0;
     if (kb0 >= L) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, lr = lane & 31;
-    const int k0w = kb0 + wave * WAVE_ROWS;
+    const int k0w = CUT ? kb0 : kb0 + wave * WAVE_ROWS, sub = CUT ? 32 * wave : 0;
     const int key = k0w + lr;
     const bool kvalid = key < L;
     const bool rope = p.cos_t != nullptr;
@@ -1023,15 +1107,15 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
     const long krow = (long)(start + (kvalid ? key : 0)) * stride;
     split_lane_row<NP>(p.qkv + krow + kcol, kvalid, h, kh, sq);
     {
-        RowStage<BLOCK_ROWS> vst;
-        fetch_rows<BLOCK_ROWS>(vst, p.qkv + (long)start * stride + vcol, stride, L, kb0);
-        commit_swz<BLOCK_ROWS, NP>(vst, Vs, sq);
+        RowStage<ROWS> vst;
+        fetch_rows<ROWS>(vst, p.qkv + (long)start * stride + vcol, stride, L, kb0);
+        commit_swz<ROWS, NP>(vst, Vs, sq);
     }
 
     int qbeg = 0, qend = L, wbeg = 0, wend = L;
     if (hw >= 0) {
         qbeg = max(0, kb0 - hw);
-        qend = min(L, kb0 + BLOCK_ROWS + hw);
+        qend = min(L, kb0 + ROWS + hw);
         wbeg = max(0, k0w - hw);
         wend = min(L, k0w + WAVE_ROWS + hw);
     }
@@ -1069,31 +1153,32 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
         __syncthreads();
         if (qt0 + BT < qend) fetch(qt0 + BT);  // block-uniform
         // Wave-uniform: outside this wave's window, or a wave whose keys all lie past the segment end.
-        if (qt0 >= wend || qt0 + BT <= wbeg || k0w >= L) continue;
+        const int qs0 = qt0 + sub;  // the wave's 32 queries
+        if (qs0 >= wend || qs0 + 32 <= wbeg || k0w >= L) continue;
         // S[q][key] = Q·Kᵀ and dP = dO·Vᵀ: lane column = its key, rows = 16 queries.
         f32x16 s = f32x16{}, dp = f32x16{};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             V8 f[NP], vh[NP];
-            swz_row_frag<BT, NP>(Qs, lr, ks, h, f);
+            swz_row_frag<BT, NP>(Qs, sub + lr, ks, h, f);
             s = Pieces<NP>::mma(f, kh[ks], s);
-            swz_row_frag<BT, NP>(Os, lr, ks, h, f);
-            swz_row_frag<BLOCK_ROWS, NP>(Vs, wave * WAVE_ROWS + lr, ks, h, vh);
+            swz_row_frag<BT, NP>(Os, sub + lr, ks, h, f);
+            swz_row_frag<ROWS, NP>(Vs, (CUT ? 0 : wave * WAVE_ROWS) + lr, ks, h, vh);
             dp = Pieces<NP>::mma(f, vh, dp);
         }
         // dP stays in its operands' scaled units (2^(eo + eq)), the row constants were staged in the same
         // units and the units' factor sits in the softmax scale dsc, which the two-piece split applies
         // (dmul = 1) and the three-piece form multiplies in (dmul = dsc).
         float pm[16], ds[16];
-        const int rel0 = qt0 + 4 * h - win.lo;  // query − lo of the lane's row r = 0
+        const int rel0 = qs0 + 4 * h - win.lo;  // query − lo of the lane's row r = 0
         // Outside the window the exponent is −∞ and the probability exactly 0 (no branch per score).
         if constexpr (!DROP) {
-            const bool inside = subtile_inside(qt0, k0w, L, hw);
+            const bool inside = subtile_inside(qs0, k0w, L, hw);
             // The row constants of the lane's 16 queries, rows 8u + 4h … +3 for u < 4: one b128 read per u.
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const f32x4 lq = *reinterpret_cast<const f32x4*>(lse_s + 8 * u + 4 * h);
-                const f32x4 dq4 = *reinterpret_cast<const f32x4*>(dot_s + 8 * u + 4 * h);
+                const f32x4 lq = *reinterpret_cast<const f32x4*>(lse_s + sub + 8 * u + 4 * h);
+                const f32x4 dq4 = *reinterpret_cast<const f32x4*>(dot_s + sub + 8 * u + 4 * h);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int r = 4 * u + i;
@@ -1105,7 +1190,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int ql = 8 * (r >> 2) + 4 * h + (r & 3);
+                const int ql = sub + 8 * (r >> 2) + 4 * h + (r & 3);
                 const bool ok = in_range(win, rel0 + 8 * (r >> 2) + (r & 3));
                 const float pr = fast_exp2(ok ? s[r] * scale_log2 - lse_s[ql] : NEG_INF);
                 const float drop =
@@ -1129,14 +1214,30 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt) {
                 V8 f[NP];
-                swz_col_frag<BT, NP>(Os, 16 * u, dt, lane, f);
+                swz_col_frag<BT, NP>(Os, sub + 16 * u, dt, lane, f);
                 dv[dt] = Pieces<NP>::mma(f, ph, dv[dt]);
-                swz_col_frag<BT, NP>(Qs, 16 * u, dt, lane, f);
+                swz_col_frag<BT, NP>(Qs, sub + 16 * u, dt, lane, f);
                 dk[dt] = Pieces<NP>::mma(f, dh, dk[dt]);
             }
         }
     }
 
+    if constexpr (CUT) {
+        float* red_k = reinterpret_cast<float*>(Qs);  // [wave][accumulator register][lane]
+        float* red_v = reinterpret_cast<float*>(Os);
+        __syncthreads();
+        park(red_k, wave, lane, dk, ldexpf(1.0f, -(eds + eq)));
+        park(red_v, wave, lane, dv, ldexpf(1.0f, -(ep + eo)));
+        __syncthreads();
+        unsigned am = 0;
+        if (kvalid) {
+            float* dst = p.dqkv + (long)(start + key) * stride;
+            am = max(store_parked(red_k, lane, wave, p, rope, key, dst + kcol),
+                     store_parked(red_v, lane, wave, p, false, key, dst + vcol));
+        }
+        block_amax_fold(am, p.amax);
+        return;
+    }
     // The epilogue's lane values are taken again after the loop rather than held across it.
     int te = threadIdx.x;
     asm volatile("" : "+v"(te));
@@ -1153,20 +1254,23 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_x6_kernel(Params p) {
 
 // Each wave owns 32 queries: q split once into registers, dO split once into the block's LDS planes (each
 // wave reads back only its own rows), which keeps the two-piece form within three waves per SIMD.
-template <int D, bool DROP, int NP = 3>
-__global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kernel(Params p) {
+template <int D, bool DROP, int NP = 3, int ROWS = BLOCK_ROWS>
+__global__ __launch_bounds__(THREADS, ROWS != BLOCK_ROWS ? 1 : NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kernel(Params p) {
     static_assert(D == 64, "split-product attention is written for head_dim 64");
+    constexpr bool CUT = ROWS == WAVE_ROWS;  // few rows: the waves share their queries and take a key subtile each
+    static_assert(!CUT || NP == 2, "the shared form is written for two-piece products");
+    constexpr int BT = CUT ? CUT_TILE : laya::BT;
     __shared__ __attribute__((aligned(16))) __bf16 Ks[NP * BT * 64];  // K tile, swizzled [key][d]
     __shared__ __attribute__((aligned(16))) __bf16 Vs[NP * BT * 64];  // V tile, swizzled [key][d]
-    __shared__ __attribute__((aligned(16))) __bf16 Ob[NP * BLOCK_ROWS * 64];  // the block's dO rows, swizzled
+    __shared__ __attribute__((aligned(16))) __bf16 Ob[NP * ROWS * 64];  // the block's dO rows, swizzled
 
-    const BlockCoord bc = block_coord(p);
+    const BlockCoord bc = block_coord<ROWS>(p);
     const int seg = bc.seg, head = bc.head;
     const int start = p.seg_start[seg], L = p.seg_len[seg];
     const int qb0 = bc.row0;
     if (qb0 >= L) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, lr = lane & 31;
-    const int q0w = qb0 + wave * WAVE_ROWS;
+    const int q0w = CUT ? qb0 : qb0 + wave * WAVE_ROWS, sub = CUT ? 32 * wave : 0;
     const int q = q0w + lr;
     const bool qvalid = q < L;
     const bool rope = p.cos_t != nullptr;
@@ -1198,7 +1302,7 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
     int kbeg = 0, kend = L, wbeg = 0, wend = L;
     if (hw >= 0) {
         kbeg = max(0, qb0 - hw);
-        kend = min(L, qb0 + BLOCK_ROWS + hw);
+        kend = min(L, qb0 + ROWS + hw);
         wbeg = max(0, q0w - hw);
         wend = min(L, q0w + WAVE_ROWS + hw);
     }
@@ -1211,14 +1315,15 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
 
     V8 qh[4][NP];
     qrow.split<NP>(qh, sq);
-    {
+    const int own = CUT ? 0 : wave * WAVE_ROWS;  // the wave's first row in Ob
+    if (!CUT || wave == 0) {
         V8 oh[4][NP];
         orow.split<NP>(oh, so);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
             for (int pl = 0; pl < NP; ++pl)
-                *reinterpret_cast<V8*>(Ob + pl * BLOCK_ROWS * 64 + swz(wave * WAVE_ROWS + lr, 16 * ks + 8 * h)) = oh[ks][pl];
+                *reinterpret_cast<V8*>(Ob + pl * ROWS * 64 + swz(own + lr, 16 * ks + 8 * h)) = oh[ks][pl];
     }
     // The row constant Σ_d dO·O (Ops.cs:408-409) from the lane's half of the row and its partner's, written
     // for the dK/dV kernel, which runs after this one.
@@ -1229,7 +1334,7 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
         dot += a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
     }
     dot += __shfl_xor(dot, 32, 64);
-    if (qvalid && h == 0) p.dots[(long)qs * p.heads + head] = dot;
+    if (qvalid && h == 0 && (!CUT || wave == 0)) p.dots[(long)qs * p.heads + head] = dot;
     const float dotu = NP == 2 ? ldexpf(dot, eo + eq) : dot;  // in dP's scaled units
     const float dsc = p.scale * udp;
     const float dmul = NP == 2 ? 1.0f : dsc;
@@ -1249,26 +1354,27 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
             fetch_rows<BT>(vst, vbase, stride, L, kt0 + BT);
         }
         // Wave-uniform: outside this wave's window, or a wave whose rows all lie past the segment end.
-        if (kt0 >= wend || kt0 + BT <= wbeg || q0w >= L) continue;
+        const int ks0 = kt0 + sub;  // the wave's 32 keys
+        if (ks0 >= wend || ks0 + 32 <= wbeg || q0w >= L) continue;
         // Sᵀ = K·Qᵀ and dPᵀ = V·dOᵀ: lane column = its query, rows = 16 keys.
         f32x16 s = f32x16{}, dp = f32x16{};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             V8 f[NP];
-            swz_row_frag<BT, NP>(Ks, lr, ks, h, f);
+            swz_row_frag<BT, NP>(Ks, sub + lr, ks, h, f);
             s = Pieces<NP>::mma(f, qh[ks], s);
             V8 o[NP];
-            swz_row_frag<BT, NP>(Vs, lr, ks, h, f);
-            swz_row_frag<BLOCK_ROWS, NP>(Ob, wave * WAVE_ROWS + lr, ks, h, o);
+            swz_row_frag<BT, NP>(Vs, sub + lr, ks, h, f);
+            swz_row_frag<ROWS, NP>(Ob, own + lr, ks, h, o);
             dp = Pieces<NP>::mma(f, o, dp);
         }
         // dP stays in its operands' scaled units (2^(eo + eq)); the row constant is taken into the same units
         // (dotu) and the units' factor into the softmax scale dsc, which the two-piece split applies
         // (dmul = 1) and the three-piece form multiplies in (dmul = dsc).
         float ds[16];
-        const int rel0 = kt0 + 4 * h - win.lo;  // key − lo of the lane's row r = 0
+        const int rel0 = ks0 + 4 * h - win.lo;  // key − lo of the lane's row r = 0
         if (!DROP) {
-            if (subtile_inside(q0w, kt0, L, hw)) {
+            if (subtile_inside(q0w, ks0, L, hw)) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) ds[r] = fast_exp2(s[r] * scale_log2 - lse) * (dp[r] - dotu) * dmul;
             } else {
@@ -1282,7 +1388,7 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int key = kt0 + 8 * (r >> 2) + 4 * h + (r & 3);
+                const int key = ks0 + 8 * (r >> 2) + 4 * h + (r & 3);
                 const bool ok = in_range(win, rel0 + 8 * (r >> 2) + (r & 3));
                 const float pr = fast_exp2(ok ? s[r] * scale_log2 - lse : NEG_INF);
                 const float drop =
@@ -1301,13 +1407,22 @@ __global__ __launch_bounds__(THREADS, NP == 2 ? 3 : 2) void attn_bwd_dq_x6_kerne
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt) {
                 V8 f[NP];
-                swz_col_frag<BT, NP>(Ks, 16 * u, dt, lane, f);
+                swz_col_frag<BT, NP>(Ks, sub + 16 * u, dt, lane, f);
                 dq[dt] = Pieces<NP>::mma(f, dh, dq[dt]);
             }
         }
     }
 
     unsigned am = 0;
+    if constexpr (CUT) {
+        float* red = reinterpret_cast<float*>(Ks);  // [wave][accumulator register][lane]
+        __syncthreads();
+        park(red, wave, lane, dq, ldexpf(1.0f, -(eds + eq)));
+        __syncthreads();
+        if (qvalid) am = store_parked(red, lane, wave, p, rope, q, p.dqkv + (long)(start + q) * stride + qcol);
+        block_amax_fold(am, p.amax);
+        return;
+    }
     if (qvalid) {
         if (rope) inverse_rope_acc<D>(dq, p, q, h);
         am = store_acc<D>(dq, p.dqkv + (long)(start + q) * stride + qcol, h, NP == 2 ? ldexpf(1.0f, -(eds + eq)) : 1.0f);
@@ -1389,9 +1504,21 @@ const float* rotated_qkv(laya_ctx* ctx, const AttentionArgs& a, unsigned* amax =
     return out;
 }
 
-// The attention kernels' grid: one workgroup per listed block and head, else (row blocks, segments, heads).
-dim3 block_grid(const AttentionArgs& a) {
-    if (a.blocks) return dim3((unsigned)(a.n_blocks * a.heads));
+// Whether the two-piece kernels run with 32 rows to a workgroup (the short form above), which stages the streamed
+// operand four times as often: while its workgroups find a CU each, or three CUs serve four of them and the rows to
+// stream are many. Forward and backward together, us with 128 rows and with 32: 4 x 128 tokens of 12 heads with dropout
+// (48 workgroups of 128 rows) 58.9 and 40.1, 1 x 189 59.4 and 44.3; 96 workgroups: 2 x 512 122 and 111, 1 x 1024 198
+// and 173, but 8 x 128 windowed 59 and 67; 192: 4 x 512 130 and 164.
+bool short_attention(const laya_ctx* ctx, const AttentionArgs& a) {
+    if (!a.blocks) return false;
+    const long groups = (long)a.n_blocks * a.heads;
+    return 4 * groups <= ctx->cu_count || (a.half_window < 0 && a.max_len >= 512 && 8 * groups <= 3L * ctx->cu_count);
+}
+
+// The attention kernels' grid: one workgroup per listed block and head (four in the short form), else (row blocks,
+// segments, heads).
+dim3 block_grid(const AttentionArgs& a, bool cut = false) {
+    if (a.blocks) return dim3((unsigned)(a.n_blocks * a.heads * (cut ? BLOCK_ROWS / WAVE_ROWS : 1)));
     return dim3((a.max_len + BLOCK_ROWS - 1) / BLOCK_ROWS, a.nseg, a.heads);
 }
 
@@ -1436,7 +1563,8 @@ void attention_fwd(laya_ctx* ctx, const AttentionArgs& a, float* context, float*
     p.context = context;
     p.lse = lse;
     p.amax = amax;
-    const dim3 grid = block_grid(a);
+    const bool cut = pair && short_attention(ctx, a);
+    const dim3 grid = block_grid(a, cut);
     p.context16 = split ? context16 : nullptr;
     if (pair && rot_word)
         p.amax_qkv = rot_word;
@@ -1445,7 +1573,11 @@ void attention_fwd(laya_ctx* ctx, const AttentionArgs& a, float* context, float*
     {
         ProfileScope scope(ctx, pair ? "attention_fwd_h2" : split ? "attention_fwd_x6" : "attention_fwd",
                            4.0 * a.hidden * a.keys, 0.0);
-        if (pair && p.p_drop > 0.0f)
+        if (cut && p.p_drop > 0.0f)
+            LAYA_LAUNCH((attn_fwd_x6_kernel<64, true, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+        else if (cut)
+            LAYA_LAUNCH((attn_fwd_x6_kernel<64, false, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+        else if (pair && p.p_drop > 0.0f)
             LAYA_LAUNCH((attn_fwd_x6_kernel<64, true, 2>), grid, dim3(THREADS), 0, ctx->stream, p);
         else if (pair)
             LAYA_LAUNCH((attn_fwd_x6_kernel<64, false, 2>), grid, dim3(THREADS), 0, ctx->stream, p);
@@ -1483,7 +1615,8 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
     p.dots = dots;
     const long total = (long)rows * a.hidden;
     const unsigned dot_blocks = (unsigned)((total + THREADS - 1) / THREADS);
-    const dim3 grid = block_grid(a);
+    const bool cut = pair && short_attention(ctx, a);
+    const dim3 grid = block_grid(a, cut);
     // Model flops of the backward, 8·d·Σkeys, split as the kernels do the work: dK/dV (4 products of
     // which 2 recompute the forward's) and dQ (3 products, 2 recomputed).
     const double fb = 2.0 * a.hidden * a.keys;
@@ -1497,14 +1630,22 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
         {
             // dQ first: it forms each row's Σ dO·O and writes it for dK/dV.
             ProfileScope scope(ctx, "attention_bwd_dq_h2", 2.0 * fb, 0.0);
-            if (p.p_drop > 0.0f)
+            if (cut && p.p_drop > 0.0f)
+                LAYA_LAUNCH((attn_bwd_dq_x6_kernel<64, true, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+            else if (cut)
+                LAYA_LAUNCH((attn_bwd_dq_x6_kernel<64, false, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+            else if (p.p_drop > 0.0f)
                 LAYA_LAUNCH((attn_bwd_dq_x6_kernel<64, true, 2>), grid, dim3(THREADS), 0, ctx->stream, p);
             else
                 LAYA_LAUNCH((attn_bwd_dq_x6_kernel<64, false, 2>), grid, dim3(THREADS), 0, ctx->stream, p);
             check_launch("attn_bwd_dq_x6_kernel");
         }
         ProfileScope scope(ctx, "attention_bwd_dkv_h2", 2.0 * fb, 0.0);
-        if (p.p_drop > 0.0f)
+        if (cut && p.p_drop > 0.0f)
+            LAYA_LAUNCH((attn_bwd_dkv_x6_kernel<64, true, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+        else if (cut)
+            LAYA_LAUNCH((attn_bwd_dkv_x6_kernel<64, false, 2, WAVE_ROWS>), grid, dim3(THREADS), 0, ctx->stream, p);
+        else if (p.p_drop > 0.0f)
             LAYA_LAUNCH((attn_bwd_dkv_x6_kernel<64, true, 2>), grid, dim3(THREADS), 0, ctx->stream, p);
         else
             LAYA_LAUNCH((attn_bwd_dkv_x6_kernel<64, false, 2>), grid, dim3(THREADS), 0, ctx->stream, p);

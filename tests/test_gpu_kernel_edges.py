@@ -99,3 +99,33 @@ def test_short_product_with_non_finite_operands(ctx):
     bad = np.isin(np.arange(96), (7, 40))
     assert not np.isfinite(y[bad]).any()
     assert _rel(y[~bad], x[~bad].astype(np.float64) @ W.astype(np.float64).T) < 1e-6
+
+
+@pytest.mark.parametrize("p_drop", [0.0, 0.2])
+@pytest.mark.parametrize("window", [-1, 64])
+@pytest.mark.parametrize("lengths", [[1], [31, 33, 1], [128], [129, 32], [189], [300, 7], [640], [513, 512]])
+def test_short_attention(ctx, lengths, window, p_drop):
+    """Attention of grids small enough for 32 rows to a workgroup (up to 64 workgroups of 128 rows; 96 without a window
+    on segments of 512 and more), where each wave takes a subtile of 32 keys or queries, and the next larger grids: row
+    counts on both sides of a subtile, of a stage of four and of several stages, with RoPE where there is no dropout.
+    Against the oracle in fp64; fp32 sums over up to 640 keys: 1e-5 relative L2, as the other attention tests hold."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    heads, hidden = 12, 768
+    rows = sum(lengths)
+    r = np.random.default_rng(rows + window)
+    qkv = r.standard_normal((rows, 3 * hidden)).astype(np.float32)
+    dctx = (1e-3 * r.standard_normal((rows, hidden))).astype(np.float32)
+    theta = 10000.0 if p_drop == 0.0 else 0.0
+    rotary = ops.Rotary(ctx, 64, theta, max(lengths)) if theta else None
+    args = (np.asarray(lengths, np.int32), heads, ops.default_scale(64), window, theta, p_drop, 11)
+    want_c = oracle.attention_forward(qkv, *args, double=True)
+    want_d = oracle.attention_backward(qkv, dctx, *args, double=True)
+    segs = ops.Segments(ctx, np.asarray(lengths, np.int32))
+    shape = ops.AttentionShape(hidden, heads, ops.default_scale(64), window, rotary, p_drop, 11)
+    q, c, l = DeviceArray.from_numpy(ctx, qkv), DeviceArray(ctx, (rows, hidden)), DeviceArray(ctx, (rows * heads,))
+    d = DeviceArray(ctx, (rows, 3 * hidden))
+    ops.attention_forward(q, segs, shape, c, l)
+    ops.attention_backward(q, segs, shape, DeviceArray.from_numpy(ctx, dctx), d, c, l)
+    assert _rel(c.numpy(), want_c) < 1e-5
+    assert _rel(d.numpy(), want_d) < 1e-5
