@@ -645,8 +645,7 @@ void column_reduce(laya_ctx* ctx, const float* part, int count, int n, float* ou
                        reinterpret_cast<const f32x4*>(part), count, w4, reinterpret_cast<f32x4*>(out));
     check_launch("colsum_reduce4_kernel");
 }
-void column_reduce_batch(laya_ctx* ctx, const ColumnSumJobs& jobs) {
-    if (jobs.n <= 0) return;
+void column_reduce_jobs(laya_ctx* ctx, const ColumnSumJobs& jobs) {
     int max_w4 = 0;
     for (int i = 0; i < jobs.n; ++i) {
         const ColumnSumJob& j = jobs.job[i];
@@ -654,11 +653,15 @@ void column_reduce_batch(laya_ctx* ctx, const ColumnSumJobs& jobs) {
                      "column_reduce_batch: 16-byte aligned rows of a multiple of 4");
         max_w4 = std::max(max_w4, j.n / 4);
     }
+    LAYA_LAUNCH(colsum_reduce4_multi_kernel, dim3((max_w4 + 15) / 16, jobs.n), dim3(256), 0, ctx->stream, jobs);
+    check_launch("colsum_reduce4_multi_kernel");
+}
+void column_reduce_batch(laya_ctx* ctx, const ColumnSumJobs& jobs) {
+    if (jobs.n <= 0) return;
     double bytes = 0;
     for (int i = 0; i < jobs.n; ++i) bytes += 4.0 * jobs.job[i].n * (jobs.job[i].count + 2);
     ProfileScope scope(ctx, "column_sums_deferred", 0.0, bytes);
-    LAYA_LAUNCH(colsum_reduce4_multi_kernel, dim3((max_w4 + 15) / 16, jobs.n), dim3(256), 0, ctx->stream, jobs);
-    check_launch("colsum_reduce4_multi_kernel");
+    column_reduce_jobs(ctx, jobs);
 }
 void rotary_apply(laya_ctx* ctx, const float* cos_t, const float* sin_t, int head_dim, float* vec, int rows,
                   const int* pos, int inverse) {
