@@ -6,7 +6,7 @@
 // RNG at head<<42 | row<<21 | key (Ops.cs:318, 355, 401), and the inverse RoPE on dq and dk
 // (Ops.cs:421-427). The kernels read q and k with RoPE (segment-local positions, Gather, Ops.cs:297-313)
 // already applied: the model's QKV projection applies it in its epilogue, and the op-level entry points
-// rotate a copy first (`rope_rows_kernel`).
+// rotate a copy of them first (`rope_rows_kernel`).
 // The forward saves each row's base-2 log-sum-exp; the backward recomputes P from it instead of
 // re-running the row softmax.
 //
@@ -37,6 +37,7 @@ constexpr float LAZY_RESCALE = 8.0f;  // log2 headroom of the split-product forw
 
 struct Params {
     const float* qkv;
+    const float* v;  // rows laid out as qkv's, whose v columns are read: qkv, or the array a rotated copy was made from
     const int* seg_start;
     const int* seg_len;
     int hidden, heads, half_window;  // half_window < 0: no window
@@ -244,7 +245,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_kernel(Params p) {
     float m = -1e30f, l = 0.0f;
 
     const float* kbase = p.qkv + (long)start * stride + kcol;
-    const float* vbase = p.qkv + (long)start * stride + vcol;
+    const float* vbase = p.v + (long)start * stride + vcol;
     PlainStage<D> kst, vst;
     fetch_plain<D>(kst, kbase, stride, L, kbeg);
     fetch_plain<D>(vst, vbase, stride, L, kbeg);
@@ -650,7 +651,7 @@ __global__ __launch_bounds__(THREADS, ROWS == BLOCK_ROWS ? 2 : 1) void attn_fwd_
     float m = -1e30f, l = 0.0f;
 
     const float* kbase = p.qkv + (long)start * stride + kcol;
-    const float* vbase = p.qkv + (long)start * stride + vcol;
+    const float* vbase = p.v + (long)start * stride + vcol;
     RowStage<TILE> kst, vst;
     fetch_rows<TILE>(kst, kbase, stride, L, kbeg);
     fetch_rows<TILE>(vst, vbase, stride, L, kbeg);
@@ -841,7 +842,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dkv_kernel(Params p) {
 
     f32x4 vv[S::G];
     const long krow = (long)(start + (kvalid ? key : 0)) * stride;
-    load_lane_row<D>(p.qkv + krow + vcol, kvalid, h, vv);
+    load_lane_row<D>(p.v + krow + vcol, kvalid, h, vv);
     {
         f32x4 kv[S::G];
         load_lane_row<D>(p.qkv + krow + kcol, kvalid, h, kv);
@@ -991,7 +992,7 @@ __global__ __launch_bounds__(THREADS, 2) void attn_bwd_dq_kernel(Params p) {
     for (int dt = 0; dt < S::ND; ++dt) dq[dt] = f32x16{};
 
     const float* kbase = p.qkv + (long)start * stride + kcol;
-    const float* vbase = p.qkv + (long)start * stride + vcol;
+    const float* vbase = p.v + (long)start * stride + vcol;
     PlainStage<D> kst, vst;
     fetch_plain<D>(kst, kbase, stride, L, kbeg);
     fetch_plain<D>(vst, vbase, stride, L, kbeg);
@@ -1108,7 +1109,7 @@ __global__ __launch_bounds__(THREADS, ROWS == BLOCK_ROWS ? 2 : 1) void attn_bwd_
     split_lane_row<NP>(p.qkv + krow + kcol, kvalid, h, kh, sq);
     {
         RowStage<ROWS> vst;
-        fetch_rows<ROWS>(vst, p.qkv + (long)start * stride + vcol, stride, L, kb0);
+        fetch_rows<ROWS>(vst, p.v + (long)start * stride + vcol, stride, L, kb0);
         commit_swz<ROWS, NP>(vst, Vs, sq);
     }
 
@@ -1307,7 +1308,7 @@ __global__ __launch_bounds__(THREADS, ROWS != BLOCK_ROWS ? 1 : NP == 2 ? 3 : 2) 
         wend = min(L, q0w + WAVE_ROWS + hw);
     }
     const float* kbase = p.qkv + (long)start * stride + kcol;
-    const float* vbase = p.qkv + (long)start * stride + vcol;
+    const float* vbase = p.v + (long)start * stride + vcol;
     RowStage<BT> kst, vst;
     fetch_rows<BT>(kst, kbase, stride, L, kbeg);
     fetch_rows<BT>(vst, vbase, stride, L, kbeg);
@@ -1430,18 +1431,37 @@ __global__ __launch_bounds__(THREADS, ROWS != BLOCK_ROWS ? 1 : NP == 2 ? 3 : 2) 
     block_amax_fold(am, p.amax);
 }
 
-// RoPE at segment-local positions on the q and k columns of one segment's qkv rows, written to `out`
-// together with an unchanged copy of v (Gather, Ops.cs:297-313). One thread per float4 unit of a row:
-// the first hidden/4 units are (d, d + D/2) pairs of q and then k, the next hidden/4 copy v.
-// amax (optional): max|written value| folded into that word group (the magnitude the two-piece kernels take
-// their scale from, in the same pass).
+// RoPE at segment-local positions on the q and k columns of one segment's qkv rows, written to `out` (Gather,
+// Ops.cs:297-313); v stays where it is, and is read only when the magnitude is wanted. One thread per float4 unit of a
+// row: the first hidden/4 units are (d, d + D/2) pairs of q and then k, the next hidden/4 are v.
+// amax (optional): max|value| of the rotated q, k and of v folded into that word group (the magnitude the two-piece
+// kernels take their scale from, in the same pass). The grid's y past the segments measures `also` (also4 float4s) into
+// also_amax: the backward's output gradient, in the same launch.
+// 14 k rows of 768: 41.7 us when v was copied too (260 MB), and 11 us for the gradient's own pass.
 __global__ void rope_rows_kernel(const float* __restrict__ qkv, const int* __restrict__ seg_start,
-                                 const int* __restrict__ seg_len, int hidden, int head_dim,
+                                 const int* __restrict__ seg_len, int nseg, int hidden, int head_dim,
                                  const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-                                 float* __restrict__ out, unsigned* amax) {
+                                 float* __restrict__ out, unsigned* amax, const float* __restrict__ also, long also4,
+                                 unsigned* also_amax) {
     const int seg = blockIdx.y;
+    if (seg >= nseg) {  // block-uniform
+        const long rank = (long)(seg - nseg) * gridDim.x + blockIdx.x, all = (long)(gridDim.y - nseg) * gridDim.x;
+        const long stride = all * blockDim.x;
+        unsigned m = 0;
+        long i = rank * blockDim.x + threadIdx.x;
+        for (; i + 3 * stride < also4; i += 4 * stride) {
+            f32x4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = ld4(also + 4 * (i + u * stride));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) m = max(m, amax_bits4(v[u]));
+        }
+        for (; i < also4; i += stride) m = max(m, amax_bits4(ld4(also + 4 * i)));
+        block_amax_fold(m, also_amax);
+        return;
+    }
     const int start = seg_start[seg], L = seg_len[seg];
-    const int units = hidden / 2;  // per row
+    const int units = amax ? hidden / 2 : hidden / 4;  // per row
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int t = (int)(idx / units), u = (int)(idx - (long)t * units);
     unsigned m = 0;
@@ -1460,10 +1480,7 @@ __global__ void rope_rows_kernel(const float* __restrict__ qkv, const int* __res
             st4(out + row + col + half, rb);
             m = max(amax_bits4(ra), amax_bits4(rb));
         } else {
-            const long col = 2L * hidden + (long)(u - hidden / 4) * 4;
-            const f32x4 v = ld4(qkv + row + col);
-            st4(out + row + col, v);
-            m = amax_bits4(v);
+            m = amax_bits4(ld4(qkv + row + 2L * hidden + (long)(u - hidden / 4) * 4));
         }
     }
     block_amax_fold(m, amax);
@@ -1472,6 +1489,7 @@ __global__ void rope_rows_kernel(const float* __restrict__ qkv, const int* __res
 Params make_params(const AttentionArgs& a) {
     Params p{};
     p.qkv = a.qkv;
+    p.v = a.qkv;
     p.seg_start = a.seg_start;
     p.seg_len = a.seg_len;
     p.blocks = a.blocks;
@@ -1488,21 +1506,29 @@ Params make_params(const AttentionArgs& a) {
     return p;
 }
 
-// The qkv the kernels read: `a.qkv` itself when RoPE is already applied (or absent), else a rotated
-// copy of its segment rows in workspace slot 4, its magnitude folded into `amax` when given.
-const float* rotated_qkv(laya_ctx* ctx, const AttentionArgs& a, unsigned* amax = nullptr) {
+// The q and k the kernels read: `a.qkv` itself when RoPE is already applied (or absent), else a rotated copy of its
+// segment rows' q and k columns in workspace slot 4, qkv's magnitude folded into `amax` when given; and then, in the
+// same launch, that of the array `also` (also_n floats, a multiple of 4, 16-byte aligned) into `also_amax`.
+const float* rotated_qkv(laya_ctx* ctx, const AttentionArgs& a, unsigned* amax = nullptr, const float* also = nullptr,
+                         long also_n = 0, unsigned* also_amax = nullptr) {
     if (a.cos_table == nullptr || a.rotated) return a.qkv;
     LAYA_REQUIRE(a.rows >= 0, "attention: row count needed to rotate q and k");
     LAYA_REQUIRE(a.hidden % 8 == 0 && (a.head_dim / 2) % 4 == 0, "attention: RoPE needs head_dim % 8 == 0");
     float* out = static_cast<float*>(ctx->workspace(4, sizeof(float) * (size_t)std::max(a.rows, 1) * 3 * a.hidden));
-    const long threads = (long)a.max_len * (a.hidden / 2);
+    const long threads = (long)a.max_len * (a.hidden / (amax ? 2 : 4));
     dim3 grid((unsigned)((threads + 255) / 256), a.nseg);
-    ProfileScope scope(ctx, "attention_rope", 0.0, 4.0 * 3.0 * a.hidden * (double)a.rows * 2.0);
-    LAYA_LAUNCH(rope_rows_kernel, grid, dim3(256), 0, ctx->stream, a.qkv, a.seg_start, a.seg_len, a.hidden,
-                       a.head_dim, a.cos_table, a.sin_table, out, amax);
+    if (also) {  // blocks of eight float4s to a thread, in whole rows of the grid
+        const long blocks = std::min(1024L, (also_n / 4 + 256 * 8 - 1) / (256 * 8));
+        grid.y += (unsigned)((blocks + grid.x - 1) / grid.x);
+    }
+    ProfileScope scope(ctx, "attention_rope", 0.0, 4.0 * a.hidden * (double)a.rows * (amax ? 5.0 : 4.0) + 4.0 * also_n);
+    LAYA_LAUNCH(rope_rows_kernel, grid, dim3(256), 0, ctx->stream, a.qkv, a.seg_start, a.seg_len, a.nseg, a.hidden,
+                       a.head_dim, a.cos_table, a.sin_table, out, amax, also, also_n / 4, also_amax);
     check_launch("rope_rows_kernel");
     return out;
 }
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Whether the two-piece kernels run with 32 rows to a workgroup (the short form above), which stages the streamed
 // operand four times as often: while its workgroups find a CU each, or three CUs serve four of them and the rows to
@@ -1607,13 +1633,18 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
     if (ar.rows < 0) ar.rows = rows;
     const bool pair = a.head_dim == 64 && split_attention(ctx) && ctx->attention_pair;
     unsigned* rot_word = pair && a.cos_table && !a.rotated ? operand_ring_word(ctx) : nullptr;
-    p.qkv = rotated_qkv(ctx, ar, rot_word);
+    const long total = (long)rows * a.hidden;
+    unsigned* do_word = nullptr;  // dO's magnitude is measured while q and k are rotated
+    if (rot_word && !(amax_do.word && *amax_do.known) && aligned16(dcontext) && ar.nseg < 60000) {
+        do_word = amax_do.word ? amax_do.word : operand_ring_word(ctx);
+        if (amax_do.word) *amax_do.known = 1;
+    }
+    p.qkv = do_word ? rotated_qkv(ctx, ar, rot_word, dcontext, total, do_word) : rotated_qkv(ctx, ar, rot_word);
     p.lse = const_cast<float*>(lse);
     p.dcontext = dcontext;
     p.dqkv = dqkv;
     float* dots = static_cast<float*>(ctx->workspace(3, sizeof(float) * (size_t)rows * a.heads));
     p.dots = dots;
-    const long total = (long)rows * a.hidden;
     const unsigned dot_blocks = (unsigned)((total + THREADS - 1) / THREADS);
     const bool cut = pair && short_attention(ctx, a);
     const dim3 grid = block_grid(a, cut);
@@ -1622,11 +1653,13 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
     const double fb = 2.0 * a.hidden * a.keys;
     if (pair) {
         p.context = const_cast<float*>(context);
-        if (rot_word)
+        if (rot_word) {
             p.amax_qkv = rot_word;
-        else
-            pair_inputs(ctx, ar, p.qkv, amax_qkv, p);
-        p.amax_do = operand_amax_ref(ctx, amax_do, 4, dcontext, rows, a.hidden, a.hidden);
+            p.amax_do = do_word ? do_word : operand_amax_ref(ctx, amax_do, 4, dcontext, rows, a.hidden, a.hidden);
+        } else {
+            operand_amax_refs(ctx, amax_qkv, a.qkv, ar.rows, 3 * a.hidden, &p.amax_qkv, amax_do, dcontext, rows,
+                              a.hidden, &p.amax_do);
+        }
         {
             // dQ first: it forms each row's Σ dO·O and writes it for dK/dV.
             ProfileScope scope(ctx, "attention_bwd_dq_h2", 2.0 * fb, 0.0);

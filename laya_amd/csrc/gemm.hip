@@ -3016,6 +3016,11 @@ const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, int slot, const float
     return word;
 }
 
+void operand_amax_refs(laya_ctx* ctx, AmaxRef ra, const float* a, int rows_a, int cols_a, const unsigned** word_a,
+                       AmaxRef rb, const float* b, int rows_b, int cols_b, const unsigned** word_b) {
+    operand_amaxes(ctx, {{ra, a, rows_a, cols_a, cols_a, word_a}, {rb, b, rows_b, cols_b, cols_b, word_b}});
+}
+
 void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K, const float* A, long lda,
           const float* B, long ldb, float* C, long ldc, const float* bias, const float* R, long ldr,
           const __bf16* A16, const __bf16* B16, AmaxRef amax_a, AmaxRef amax_b, unsigned* amax_c) {
