@@ -1675,12 +1675,14 @@ struct PairPlan {
     int tn_tiles, tn_units;  // dW tiles and K units per dW tile
     int q, r;                // nn_tiles = q·G + r
     int W;                   // total units (G·W < 2³¹, checked on the host)
+    bool rest;               // dW is shared by the workers from r on alone (those before it have a dX tile more)
     float* partial;          // [G][2][BM·BN] dW partial tiles, lane order
 };
 
 // First dW unit of worker g (the end of worker g is the start of worker g + 1).
-__device__ __forceinline__ int plan_tn_lo(const PairPlan& s, int g) {
-    return g * s.W / s.G - s.nn_units * (g * s.q + min(g, s.r));
+__host__ __device__ __forceinline__ int plan_tn_lo(const PairPlan& s, int g) {
+    if (s.rest) return g <= s.r ? 0 : (int)((long)(g - s.r) * s.tn_tiles * s.tn_units / (s.G - s.r));
+    return g * s.W / s.G - s.nn_units * (g * s.q + (g < s.r ? g : s.r));
 }
 
 __device__ __forceinline__ TileCoord unit_coord(const GemmParams& p, int t, int a, int b) {
@@ -3304,6 +3306,15 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
     s.W = (int)std::min<long>(W, 1L << 30);
     const long need_min = W / s.G - (long)(s.q + (s.r > 0 ? 1 : 0)) * s.nn_units;
     const long max_run = (W + s.G - 1) / s.G - (long)s.q * s.nn_units;
+    // A dX tile is more than a worker's share: the workers that have one more of them do no dW, and the rest share it
+    // all, while that leaves the workers at least half busy (fill). us per backward, before (128 x 128 tiles) and so:
+    // 8000 x 768 -> 2304 (fill 0.74) 392 and 245, 6000 (0.56) 308 and 242, 4500 (0.42) 191 and 226; 2500 x 3072 -> 768
+    // (0.93) 185 and 111; bf16 8000 x 768 -> 2304 224 and 143, 4500 111 and 117.
+    if (need_min < 0 && s.nn_units > 0 && 2 * W >= (long)s.G * (s.q + 1) * s.nn_units) {
+        const long dW = (long)n1 * s.tn_units, workers = s.G - s.r;
+        s.rest = true;
+        return (dW + workers - 1) / workers < s.tn_units && W < (1L << 30) && s.G <= FIXUP_MAX_WORKERS;
+    }
     return need_min >= 0 && s.nn_units > 0 && W * s.G < (1L << 31) && max_run < s.tn_units &&
            s.G <= FIXUP_MAX_WORKERS;
 }
@@ -3358,10 +3369,8 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
         check_launch("gemm_pair_wide_kernel");
     }
     long partials = 0, shared = 0;
-    const long Wt = (long)n0 * s.nn_units + (long)n1 * s.tn_units;
-    auto tn_lo = [&](long g) { return g * Wt / s.G - (long)s.nn_units * (g * s.q + std::min<long>(g, s.r)); };
     for (int g = 0; ctx->profiling && g < s.G; ++g) {
-        const long lo = tn_lo(g), hi = tn_lo(g + 1);
+        const long lo = plan_tn_lo(s, g), hi = plan_tn_lo(s, g + 1);
         for (long u = lo; u < hi;) {
             const long t = u / s.tn_units, a = u - t * s.tn_units;
             const long b = std::min<long>(s.tn_units, a + (hi - u));
@@ -3395,7 +3404,18 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
         const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
         nn.amax = amax_dx;
-        if (short_pair_pays(ctx, nn, tn)) {
+        // Against the wide pair's longest worker: about 1.7 us for a unit of a 256 x 256 x 16 fp32 product and 0.85 for
+        // a bf16 one, 15 for the fixup; short products about 27 and 20 us for 10⁹ multiply-adds (4500 x 1152 -> 768:
+        // short 117, wide 97; 1618 x 2624 -> 1024: 95 and 124).
+        const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
+        const int wt_in = (in + WT - 1) / WT;
+        PairPlan s{};
+        const bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
+                                                               (out + WT - 1) / WT * wt_in, rows, s);
+        const double units = s.rest ? (s.q + 1.0) * s.nn_units : (double)s.W / s.G;
+        const double t_wide = 15.0 + (bf16 ? 0.85 : 1.7) * units;
+        const double t_short = (bf16 ? 20e-9 : 27e-9) * rows * (double)in * out;
+        if (!(wide && t_wide < t_short) && short_pair_pays(ctx, nn, tn)) {
             short_gemm_pair(ctx, nn, tn);
             *folded = amax_dx != nullptr;
             return;
@@ -3420,7 +3440,10 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
     tn.mode = STORE;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;
     PairPlan s{};
-    if ((split || fp32 || half) && make_pair_plan(ctx, n0, out, n1, rows, s)) {
+    // Two-piece products in launches of their own rather than this plan's six bf16 ones: 2500 x 3072 -> 768 185 us and
+    // 144, 10000 x 768 -> 2304 472 and 364, 4500 x 768 -> 2304 191 and 194.
+    const bool pieces = split && (ctx->matmul_pair & 6) == 6 && operand_fast(nn.A, nn.lda, nn.vec_a, true, nn.M, nn.K);
+    if (!pieces && (split || fp32 || half) && make_pair_plan(ctx, n0, out, n1, rows, s)) {
         s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * BM * BN));
         tn.mode = ACCUMULATE;
         {

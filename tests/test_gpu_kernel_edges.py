@@ -129,3 +129,26 @@ def test_short_attention(ctx, lengths, window, p_drop):
     ops.attention_backward(q, segs, shape, DeviceArray.from_numpy(ctx, dctx), d, c, l)
     assert _rel(c.numpy(), want_c) < 1e-5
     assert _rel(d.numpy(), want_d) < 1e-5
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("rows,fan_in,fan_out", [(2500, 3072, 768), (5300, 768, 2304), (6001, 768, 768)])
+def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in, fan_out):
+    """The wide backward pair where a dX tile is more than a worker's share, so that the workers with one more dX tile
+    do no dW: against fp64 on the same operands, 1e-6 relative L2 widened by the square root of K over 768 for dW, whose
+    sums run over the rows."""
+    from laya_amd import ops
+    from laya_amd.device import Context, DeviceArray
+    c = ctx if precision == "fp32" else Context(0)
+    c.set_matmul_precision(precision)
+    r = np.random.default_rng(rows)
+    x = r.standard_normal((rows, fan_in)).astype(np.float32)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
+    low = (lambda a: _bf16(a).astype(np.float64)) if precision == "bf16" else (lambda a: a.astype(np.float64))
+    Wp, dx = ops.Parameter(c, "W", W), DeviceArray(c, (rows, fan_in))
+    ops.linear_backward(Wp, None, DeviceArray.from_numpy(c, x), DeviceArray.from_numpy(c, dy), rows, dx)
+    assert _rel(dx.numpy(), low(dy) @ low(W)) < 1e-6
+    assert _rel(Wp.gradient_buffer().numpy(), low(dy).T @ low(x)) < 1e-6 * np.sqrt(rows / 768)
+    if c is not ctx:
+        c.close()
