@@ -3440,10 +3440,7 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
     tn.mode = STORE;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;
     PairPlan s{};
-    // Two-piece products in launches of their own rather than this plan's six bf16 ones: 2500 x 3072 -> 768 185 us and
-    // 144, 10000 x 768 -> 2304 472 and 364, 4500 x 768 -> 2304 191 and 194.
-    const bool pieces = split && (ctx->matmul_pair & 6) == 6 && operand_fast(nn.A, nn.lda, nn.vec_a, true, nn.M, nn.K);
-    if (!pieces && (split || fp32 || half) && make_pair_plan(ctx, n0, out, n1, rows, s)) {
+    if ((split || fp32 || half) && make_pair_plan(ctx, n0, out, n1, rows, s)) {
         s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * BM * BN));
         tn.mode = ACCUMULATE;
         {

@@ -152,3 +152,24 @@ def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in,
     assert _rel(Wp.gradient_buffer().numpy(), low(dy).T @ low(x)) < 1e-6 * np.sqrt(rows / 768)
     if c is not ctx:
         c.close()
+
+
+@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700)])
+def test_backward_pairs_on_exact_splits_keep_small_rows(ctx, rows, fan_in, fan_out):
+    """fp32 backward pairs that run as exact three-piece splits: dY rows 2^-26 below the rest, each of which a two-piece
+    product under a scale of the others would keep to about 2^(26-39) = 1e-4, come out to fp32 precision (a sum of K
+    terms rounded 2^-24 each: 2e-6 holds K = 700)."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    r = np.random.default_rng(rows + fan_out)
+    x = r.standard_normal((rows, fan_in)).astype(np.float32)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
+    dy[7::50] *= np.float32(2.0 ** -26)
+    Wp, dx = ops.Parameter(ctx, "W", W), DeviceArray(ctx, (rows, fan_in))
+    ctx.profile_begin()
+    ops.linear_backward(Wp, None, DeviceArray.from_numpy(ctx, x), DeviceArray.from_numpy(ctx, dy), rows, dx)
+    assert "gemm_bwd_pair_x6" in ctx.profile_end()
+    want = dy.astype(np.float64) @ W.astype(np.float64)
+    assert (np.linalg.norm(dx.numpy() - want, axis=1) / np.linalg.norm(want, axis=1)).max() < 2e-6
+    assert _rel(Wp.gradient_buffer().numpy(), dy.astype(np.float64).T @ x.astype(np.float64)) < 1e-6 * np.sqrt(rows / 768)
