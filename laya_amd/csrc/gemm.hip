@@ -3292,8 +3292,8 @@ bool make_pair_plan(const laya_ctx* ctx, int n0, int out, int n1, int rows, Pair
            s.G <= FIXUP_MAX_WORKERS;
 }
 
-// The same schedule over one worker per CU, 256 x 256 tiles and 16-deep units (the wide pair).
-bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows, PairPlan& s) {
+// The same schedule over one worker per CU, 256 x 256 tiles and 16-deep units (the wide pair); half: of bf16 products.
+bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows, bool half, PairPlan& s) {
     s = PairPlan{};
     s.G = ctx->cu_count;
     s.nn_tiles = n0;
@@ -3307,10 +3307,11 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
     const long need_min = W / s.G - (long)(s.q + (s.r > 0 ? 1 : 0)) * s.nn_units;
     const long max_run = (W + s.G - 1) / s.G - (long)s.q * s.nn_units;
     // A dX tile is more than a worker's share: the workers that have one more of them do no dW, and the rest share it
-    // all, while that leaves the workers at least half busy (fill). us per backward, before (128 x 128 tiles) and so:
-    // 8000 x 768 -> 2304 (fill 0.74) 392 and 245, 6000 (0.56) 308 and 242, 4500 (0.42) 191 and 226; 2500 x 3072 -> 768
-    // (0.93) 185 and 111; bf16 8000 x 768 -> 2304 224 and 143, 4500 111 and 117.
-    if (need_min < 0 && s.nn_units > 0 && 2 * W >= (long)s.G * (s.q + 1) * s.nn_units) {
+    // all, while that leaves the workers at least half busy (fill): bf16 8000 x 768 -> 2304 (fill 0.74) 224 us on 128 x
+    // 128 tiles and 143 so, 4500 (0.42) 111 and 117. Not for fp32 products: most of these shapes run as exact
+    // three-piece splits (make_pair_plan), which keep rows of dY far below its largest that two pieces under one scale
+    // would round away, and three-piece units take twice as long here.
+    if (half && need_min < 0 && s.nn_units > 0 && 2 * W >= (long)s.G * (s.q + 1) * s.nn_units) {
         const long dW = (long)n1 * s.tn_units, workers = s.G - s.r;
         s.rest = true;
         return (dW + workers - 1) / workers < s.tn_units && W < (1L << 30) && s.G <= FIXUP_MAX_WORKERS;
@@ -3335,7 +3336,7 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
     tn.tiles_n = (in + WT - 1) / WT;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;
     PairPlan s{};
-    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, s)) return false;
+    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, half, s)) return false;
     s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * WT * WT));
     const bool pair = !half && (ctx->matmul_pair & 6) == 6;
     if (pair) {
@@ -3411,7 +3412,7 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         const int wt_in = (in + WT - 1) / WT;
         PairPlan s{};
         const bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
-                                                               (out + WT - 1) / WT * wt_in, rows, s);
+                                                               (out + WT - 1) / WT * wt_in, rows, bf16, s);
         const double units = s.rest ? (s.q + 1.0) * s.nn_units : (double)s.W / s.G;
         const double t_wide = 15.0 + (bf16 ? 0.85 : 1.7) * units;
         const double t_short = (bf16 ? 20e-9 : 27e-9) * rows * (double)in * out;

@@ -154,11 +154,11 @@ def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in,
         c.close()
 
 
-@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700)])
+@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700), (2500, 3072, 768), (8003, 768, 2304)])
 def test_backward_pairs_on_exact_splits_keep_small_rows(ctx, rows, fan_in, fan_out):
     """fp32 backward pairs that run as exact three-piece splits: dY rows 2^-26 below the rest, each of which a two-piece
     product under a scale of the others would keep to about 2^(26-39) = 1e-4, come out to fp32 precision (a sum of K
-    terms rounded 2^-24 each: 2e-6 holds K = 700)."""
+    terms rounded 2^-24 each: 2e-6 holds K = 2304)."""
     from laya_amd import ops
     from laya_amd.device import DeviceArray
     r = np.random.default_rng(rows + fan_out)
