@@ -3416,7 +3416,13 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         const double units = s.rest ? (s.q + 1.0) * s.nn_units : (double)s.W / s.G;
         const double t_wide = 15.0 + (bf16 ? 0.85 : 1.7) * units;
         const double t_short = (bf16 ? 20e-9 : 27e-9) * rows * (double)in * out;
-        if (!(wide && t_wide < t_short) && short_pair_pays(ctx, nn, tn)) {
+        // Nor where an fp32 pair runs as exact three-piece splits, the balanced plan below (5600 x 768 -> 768): two
+        // pieces would keep rows of dY far below its largest to fewer bits.
+        PairPlan exact{};
+        const bool pieces3 = !bf16 && !wide &&
+                             make_pair_plan(ctx, (rows + BM - 1) / BM * ((in + BN - 1) / BN), out,
+                                            (out + BM - 1) / BM * ((in + BN - 1) / BN), rows, exact);
+        if (!(wide && t_wide < t_short) && !pieces3 && short_pair_pays(ctx, nn, tn)) {
             short_gemm_pair(ctx, nn, tn);
             *folded = amax_dx != nullptr;
             return;

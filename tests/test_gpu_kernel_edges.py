@@ -154,7 +154,8 @@ def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in,
         c.close()
 
 
-@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700), (2500, 3072, 768), (8003, 768, 2304)])
+@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700), (2500, 3072, 768), (8003, 768, 2304),
+                                                 (1400, 3072, 768), (5600, 768, 768), (1600, 2624, 1024)])
 def test_backward_pairs_on_exact_splits_keep_small_rows(ctx, rows, fan_in, fan_out):
     """fp32 backward pairs that run as exact three-piece splits: dY rows 2^-26 below the rest, each of which a two-piece
     product under a scale of the others would keep to about 2^(26-39) = 1e-4, come out to fp32 precision (a sum of K
