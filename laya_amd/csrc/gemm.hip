@@ -2994,6 +2994,33 @@ int fill_splits(const laya_ctx* ctx, int tiles, int K, int min_k) {
     return std::max(1, std::min({slots / tiles, K / min_k, 32}));
 }
 
+// Microseconds that measuring a product's operands adds: one launch over those whose magnitude is not known.
+double measuring_time(std::initializer_list<std::pair<AmaxRef, double>> operands) {
+    double bytes = 0.0;
+    for (const auto& [ref, elements] : operands)
+        if (!ref.word || !*ref.known) bytes += 4.0 * elements;
+    return bytes > 0.0 ? 3.3 + 0.14e-6 * bytes : 0.0;
+}
+
+// Microseconds a product takes on the tiles of this file, its operands' magnitudes known, as the short products of
+// gemm_short.hip are weighed against: 128 x 128 tiles with K split over idle CUs, the partials written and summed.
+// Fitted to the same shapes as theirs, where it is within 20 % for four in five; the 256-wide tiles that the larger of
+// them take come out near it.
+double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16) {
+    const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    GemmParams p{};
+    p.K = K;
+    const int splits = set_splits(p, fill_splits(ctx, tiles, K, 128));
+    const long slots = 2L * ctx->cu_count, rounds = ((long)tiles * splits + slots - 1) / slots;
+    const double mb = 4e-6 * M * N;
+    return 7.0 + (bf16 ? 0.75 : 1.3) * rounds * (p.k_per_split / BK) + (splits > 1 ? 0.45 * splits * mb : 0.0) + 0.2 * mb;
+}
+
+// The same with the time its operands' magnitudes take (A is M x K and B N x K, however they are stored).
+double product_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, AmaxRef a, AmaxRef b) {
+    return tiles_time(ctx, M, N, K, bf16) + (bf16 ? 0.0 : measuring_time({{a, (double)M * K}, {b, (double)N * K}}));
+}
+
 }  // namespace
 
 // Each half of the ring is cleared, in one launch, as the measurements enter it.
@@ -3032,7 +3059,8 @@ void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K
         g.amax = amax_c;
         const ShortEpilogue se =
             ep == GemmEpilogue::Store ? ShortEpilogue::Store : ShortEpilogue::Accumulate;
-        if (short_gemm_pays(ctx, layout, se, g)) {
+        const int cls = layout == GemmLayout::NT ? 1 : layout == GemmLayout::NN ? 2 : 4;
+        if (short_gemm_pays(ctx, layout, se, g, product_time(ctx, M, N, K, ctx->matmul_bf16 & cls, amax_a, amax_b))) {
             short_gemm(ctx, layout, se, g);
             return;
         }
@@ -3123,7 +3151,9 @@ void gemm_rope(laya_ctx* ctx, int M, int N, int K, const float* A, const float* 
     g.rope_cos = cos_t;
     g.rope_sin = sin_t;
     g.rope_cols = rope_cols;
-    if (rope_cols <= N && pos && cos_t && sin_t && short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Rope, g)) {
+    const double tiles_us = product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_a, amax_b);
+    if (rope_cols <= N && pos && cos_t && sin_t &&
+        short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Rope, g, tiles_us)) {
         short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Rope, g);
         return;
     }
@@ -3222,7 +3252,10 @@ void gemm_geglu(laya_ctx* ctx, int M, int inter, int K, const float* x, const fl
     g.act = act;
     g.act16 = act16;
     g.inter = inter;
-    if (short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g)) {
+    // Against the product and a GeGLU pass over its output (12 bytes a value of act, at 5 TB/s).
+    const double geglu_us = 4.0 + 0.2 * 12e-6 * M * inter;
+    if (short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g,
+                        product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_x, amax_W) + geglu_us)) {
         short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g);
         return;
     }
@@ -3405,24 +3438,29 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
         const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
         nn.amax = amax_dx;
-        // Against the wide pair's longest worker: about 1.7 us for a unit of a 256 x 256 x 16 fp32 product and 0.85 for
-        // a bf16 one, 15 for the fixup; short products about 27 and 20 us for 10⁹ multiply-adds (4500 x 1152 -> 768:
-        // short 117, wide 97; 1618 x 2624 -> 1024: 95 and 124).
+        // Against the wide pair's longest worker and its fixup, us fitted to 60 shapes each (a unit is a 256 x 256 x 16
+        // product), or dX and dW in launches of their own, less what the second saves by following the first.
         const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
-        const int wt_in = (in + WT - 1) / WT;
+        const int wt_in = (in + WT - 1) / WT, t_in = (in + BN - 1) / BN;
         PairPlan s{};
         const bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
                                                                (out + WT - 1) / WT * wt_in, rows, bf16, s);
-        const double units = s.rest ? (s.q + 1.0) * s.nn_units : (double)s.W / s.G;
-        const double t_wide = 15.0 + (bf16 ? 0.85 : 1.7) * units;
-        const double t_short = (bf16 ? 20e-9 : 27e-9) * rows * (double)in * out;
+        double other;
+        if (wide && s.rest)
+            other = 25.0 + 0.75 * std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
+        else if (wide)
+            other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
+        else
+            other = (bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
+                    (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16);
+        if (!bf16)
+            other += measuring_time({{amax_dy, (double)rows * out}, {amax_W, (double)out * in}, {amax_x, (double)rows * in}});
         // Nor where an fp32 pair runs as exact three-piece splits, the balanced plan below (5600 x 768 -> 768): two
         // pieces would keep rows of dY far below its largest to fewer bits.
         PairPlan exact{};
         const bool pieces3 = !bf16 && !wide &&
-                             make_pair_plan(ctx, (rows + BM - 1) / BM * ((in + BN - 1) / BN), out,
-                                            (out + BM - 1) / BM * ((in + BN - 1) / BN), rows, exact);
-        if (!(wide && t_wide < t_short) && !pieces3 && short_pair_pays(ctx, nn, tn)) {
+                             make_pair_plan(ctx, (rows + BM - 1) / BM * t_in, out, (out + BM - 1) / BM * t_in, rows, exact);
+        if (!pieces3 && short_pair_pays(ctx, nn, tn, other)) {
             short_gemm_pair(ctx, nn, tn);
             *folded = amax_dx != nullptr;
             return;

@@ -458,34 +458,103 @@ bool short_gemm_fits(const ShortGemm& g, GemmLayout layout, ShortEpilogue ep) {
     return true;
 }
 
-// Up to how many multiply-adds a product runs here. Measured against gemm.hip's tiles, us there and here, fp32 with the
-// operands' magnitudes measured there: forward 404 x 1024 -> 3072 32 and 19, 1618 x 768 -> 2304 (2.9e9) 44 and 37, 2200
-// rows (3.9e9) 52 and 48, 3200 rows (5.7e9) 54 and 73; the backward pair 512 x 768 -> 2304 61 and 26, 1618 x 1024 ->
-// 2624 (4.3e9) 150 and 107, 3200 x 768 -> 2304 (5.7e9) 145 and 139 (slower here where the magnitudes are known), 3200 x
-// 3072 -> 768 (7.5e9) 155 and 186. bf16 products have no magnitudes to measure and less to split there: forward 1100 x
-// 768 -> 2304 (1.9e9) 24 and 23, the pair 1618 x 768 -> 2304 (2.9e9) 59 and 55, 1618 x 3072 -> 768 (3.8e9) 66 and 69;
-// 60 x 1024 -> 5248, whose dX is sixteen tiles of a long K, 27 and 35.
+// Up to how many multiply-adds a product may run here: the range over which the times below were fitted.
 constexpr double FORWARD_LIMIT = 4.0e9, FORWARD_LIMIT_BF16 = 2.0e9, PAIR_LIMIT = 5.0e9, PAIR_LIMIT_BF16 = 3.0e9;
-constexpr int PAIR_OUT_BF16 = 4096;
 
 double work_of(const ShortGemm& g) { return (double)g.M * g.N * g.K; }
 
-}  // namespace
+bool is_bf16(const laya_ctx* ctx, GemmLayout layout) { return ctx->matmul_bf16 & layout_class(layout); }
 
-bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g) {
-    const int cls = layout_class(layout);
-    const bool bf16 = ctx->matmul_bf16 & cls;
-    if (!bf16 && !((ctx->matmul_pair & cls) && (ctx->matmul_split & cls))) return false;
-    return work_of(g) <= (bf16 ? FORWARD_LIMIT_BF16 : FORWARD_LIMIT) && short_gemm_fits(g, layout, ep);
+// A product's tiles and how many waves share one.
+struct Shape {
+    int tm, tn, waves;
+    long tiles;
+};
+
+// Smaller tiles while they would leave nearly half the CUs without one (404 x 3072 -> 768: 84 tiles of 64 x 64
+// 27.6 us, 156 of 32 x 64 21.0, 312 of 32 x 32 25.9; 800 x 768 -> 768, 156 tiles: 11.6, 14.1 with 32 x 64). Past a
+// tile per CU workgroups of four waves, two to a CU, hide each other's first loads and epilogues (1618 x 768 -> 2304
+// 47.8 us with eight waves, 36.9 with four); under it eight waves shorten each one's K (3072 -> 768 27.6 and 34.8).
+Shape shape_of(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g) {
+    const long few = ctx->cu_count * 9L / 16;
+    Shape s{64, 64, 8, 0};
+    if (layout == GemmLayout::NT) {
+        if (tiles_of(g, ep, s.tm, s.tn) < few) s.tm = 32;
+        if (ep == ShortEpilogue::Store && tiles_of(g, ep, s.tm, s.tn) < few) s.tn = 32;
+    }
+    s.tiles = tiles_of(g, ep, s.tm, s.tn);
+    if (s.tm == 64 && s.tiles > ctx->cu_count) s.waves = 4;
+    return s;
 }
 
-bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) {
+long ceil_div(long a, long b) { return (a + b - 1) / b; }
+
+// The stages a wave goes through, one after the other.
+long chain_of(const ShortGemm& g, int waves) { return ceil_div(ceil_div(g.K, UNIT), waves); }
+
+double megabytes(double floats) { return 4e-6 * floats; }
+
+// Microseconds a product takes here: its rounds of workgroups, each a chain of stages and an epilogue. Work alone does
+// not say it: dW of 768 x 64 over 65,536 rows is twelve workgroups of 256 stages a wave, 460 us here and 130 with K split
+// over the chip; 65536 x 64 -> 768 forward is 12,288 tiles of half a stage a wave, 109 us here and 65 on 256-wide tiles.
+// Fitted to 250 shapes per precision (widths 32 … 4096, 16 … 131,072 rows, back to back on one stream), where it is
+// within 15 % for four in five. Choosing by it and by the other tiles' estimate was within 2 % of the faster of the two
+// in sum over 290 other shapes, forward, dX, dW and pair alike.
+double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g) {
+    const bool bf16 = is_bf16(ctx, layout), nt = layout == GemmLayout::NT;
+    const Shape s = shape_of(ctx, layout, ep, g);
+    const bool small = s.tn == 32;
+    double stage;
+    if (small) stage = bf16 ? 0.34 : 0.87;
+    else if (s.tm == 32) stage = bf16 ? 0.87 : 1.55;
+    else if (s.waves == 4) stage = bf16 ? 1.45 : 2.15;
+    else stage = nt ? (bf16 ? 1.65 : 2.4) : bf16 ? 1.1 : 1.9;
+    const long per_round = (s.waves == 4 || small ? 2L : 1L) * ctx->cu_count;
+    return 2.5 + ceil_div(s.tiles, per_round) * (2.0 + stage * chain_of(g, s.waves)) +
+           (ep == ShortEpilogue::Accumulate ? 0.25 : 0.05) * megabytes((double)g.M * g.N);
+}
+
+// As for the forward; and eight waves where dX is few tiles of a long K, which last longest (512 x 768 -> 2304, 96
+// tiles: 27 us with eight waves, 32 with four; 800 rows, 156 tiles: 41 and 36).
+int pair_waves(const laya_ctx* ctx, const ShortGemm& nn, long dx_tiles, long dw_tiles) {
+    return dx_tiles + dw_tiles > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048) ? 4 : 8;
+}
+
+// The same of a pair: dX's workgroups, then dW's. Where they come in more than one round the last of dW's begin, on the
+// average, half their length before the others are done.
+double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) {
+    const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
+    const long dx = tiles_of(nn, ShortEpilogue::Store, 64, 64), dw = tiles_of(tn, ShortEpilogue::Accumulate, 64, 64);
+    const int waves = pair_waves(ctx, nn, dx, dw);
+    const long slots = (waves == 4 ? 2L : 1L) * ctx->cu_count;
+    const double epilogue = bf16 ? 1.7 : 1.0, stage = bf16 ? (waves == 4 ? 1.3 : 1.15) : waves == 4 ? 1.95 : 1.9;
+    const double a = chain_of(nn, waves) + epilogue, b = chain_of(tn, waves) + epilogue;
+    double span = std::max(a, b);
+    if (dx + dw > slots) span = std::max(span, (dx * a + dw * b) / slots + 0.5 * b);
+    return 4.0 + stage * span;
+}
+
+// A product runs here only where the estimates differ by more than this; bf16 ones scatter more (3200 x 1152 -> 768, the
+// pair: 50 and 59 estimated, 68 and 56 measured).
+constexpr double MARGIN = 0.95, MARGIN_BF16 = 0.9;
+
+}  // namespace
+
+bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g, double other) {
+    const int cls = layout_class(layout);
+    const bool bf16 = is_bf16(ctx, layout);
+    if (!bf16 && !((ctx->matmul_pair & cls) && (ctx->matmul_split & cls))) return false;
+    return work_of(g) <= (bf16 ? FORWARD_LIMIT_BF16 : FORWARD_LIMIT) && short_gemm_fits(g, layout, ep) &&
+           short_time(ctx, layout, ep, g) < (bf16 ? MARGIN_BF16 : MARGIN) * other;
+}
+
+bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, double other) {
     const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
     if (!bf16 && ((ctx->matmul_bf16 & 6) || (ctx->matmul_pair & 6) != 6 || (ctx->matmul_split & 6) != 6)) return false;
-    if (bf16 && nn.K > PAIR_OUT_BF16) return false;
     return work_of(nn) <= (bf16 ? PAIR_LIMIT_BF16 : PAIR_LIMIT) &&
            short_gemm_fits(nn, GemmLayout::NN, ShortEpilogue::Store) &&
-           short_gemm_fits(tn, GemmLayout::TN, ShortEpilogue::Accumulate);
+           short_gemm_fits(tn, GemmLayout::TN, ShortEpilogue::Accumulate) &&
+           pair_time(ctx, nn, tn) < (bf16 ? MARGIN_BF16 : MARGIN) * other;
 }
 
 #define SHORT_NP(W, ...)                                                                                   \
@@ -501,23 +570,15 @@ void short_gemm(laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, ShortGemm g)
                    GE = ShortEpilogue::Geglu;
     LAYA_REQUIRE(layout == GemmLayout::NT ? ep != AC : ep == (layout == GemmLayout::NN ? ST : AC),
                  "short_gemm: no such product");
-    const bool bf16 = ctx->matmul_bf16 & layout_class(layout);
+    const bool bf16 = is_bf16(ctx, layout);
     static const char* names[3][2] = {{"gemm_nt_h2s", "gemm_nt_bf16s"},
                                       {"gemm_nn_h2s", "gemm_nn_bf16s"},
                                       {"gemm_tn_h2s", "gemm_tn_bf16s"}};
-    // Smaller tiles while they would leave nearly half the CUs without one (404 x 3072 -> 768: 84 tiles of 64 x 64
-    // 27.6 us, 156 of 32 x 64 21.0, 312 of 32 x 32 25.9; 800 x 768 -> 768, 156 tiles: 11.6, 14.1 with 32 x 64). Past a
-    // tile per CU workgroups of four waves, two to a CU, hide each other's first loads and epilogues (1618 x 768 -> 2304
-    // 47.8 us with eight waves, 36.9 with four); under it eight waves shorten each one's K (3072 -> 768 27.6 and 34.8).
-    const long few = ctx->cu_count * 9L / 16;
-    int tm = 64, tn = 64;
-    if (layout == GemmLayout::NT) {
-        if (tiles_of(g, ep, tm, tn) < few) tm = 32;
-        if (ep == ST && tiles_of(g, ep, tm, tn) < few) tn = 32;
-    }
+    const Shape s = shape_of(ctx, layout, ep, g);
+    const int tm = s.tm, tn = s.tn;
     set_tiles(g, ep, tm, tn);
     const dim3 grid(g.tiles_m * g.tiles_n);
-    const bool w4 = tm == 64 && (long)grid.x > ctx->cu_count;
+    const bool w4 = s.waves == 4;
     ProfileScope scope(ctx, names[(int)layout][bf16], 2.0 * g.M * g.N * (double)g.K, 0.0);
     if (layout == GemmLayout::NT) {
         if (ep == RO && w4) SHORT_NP(4, true, true, 64, 64, RO);
@@ -547,9 +608,7 @@ void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn) {
     set_tiles(tn, ShortEpilogue::Accumulate, 64, 64);
     const int dx_tiles = nn.tiles_m * nn.tiles_n;
     const dim3 grid(dx_tiles + tn.tiles_m * tn.tiles_n);
-    // As for the forward; and eight waves where dX is few tiles of a long K, which last longest (512 x 768 -> 2304, 96
-    // tiles: 27 us with eight waves, 32 with four; 800 rows, 156 tiles: 41 and 36).
-    const bool w4 = (long)grid.x > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048);
+    const bool w4 = pair_waves(ctx, nn, dx_tiles, (long)grid.x - dx_tiles) == 4;
     ProfileScope scope(ctx, bf16 ? "gemm_bwd_pair_bf16s" : "gemm_bwd_pair_h2s", 4.0 * nn.M * nn.N * (double)nn.K, 0.0);
 #define SHORT_PAIR(W, NP) \
     LAYA_LAUNCH((short_pair_kernel<W, NP>), grid, dim3(64 * W), 0, ctx->stream, nn, tn, dx_tiles)

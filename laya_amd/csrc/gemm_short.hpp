@@ -26,12 +26,12 @@ struct ShortGemm {
     int tiles_m, tiles_n;  // set by the launchers
 };
 
-// Whether the product runs here (its shape allows it and these tiles take less time than gemm.hip's), under the
-// context's precision for its layout: two-piece fp16 products, or bf16 operands.
-bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g);
+// Whether the product runs here, under the context's precision for its layout (two-piece fp16 products, or bf16
+// operands): its shape allows it and these tiles take less time than `other`, gemm.hip's in microseconds.
+bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g, double other);
 void short_gemm(laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, ShortGemm g);
 // A linear layer's dX (NN, Store) and dW (TN, Accumulate) in one launch.
-bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn);
+bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, double other);
 void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn);
 
 }  // namespace laya

@@ -174,3 +174,50 @@ def test_backward_pairs_on_exact_splits_keep_small_rows(ctx, rows, fan_in, fan_o
     want = dy.astype(np.float64) @ W.astype(np.float64)
     assert (np.linalg.norm(dx.numpy() - want, axis=1) / np.linalg.norm(want, axis=1)).max() < 2e-6
     assert _rel(Wp.gradient_buffer().numpy(), dy.astype(np.float64).T @ x.astype(np.float64)) < 1e-6 * np.sqrt(rows / 768)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("rows,fan_in,fan_out,short", [
+    (13824, 768, 64, "forward"), (32768, 64, 768, "dx"), (32768, 64, 64, "forward dx"), (8192, 256, 256, "forward dx"),
+    (8192, 768, 32, "forward"), (404, 768, 768, "forward dx dw pair"), (512, 768, 2304, "forward dx dw pair")])
+def test_short_products_only_where_they_fill_the_chip(ctx, precision, rows, fan_in, fan_out, short):
+    """Narrow layers over many rows: a dW of a few tiles and a long K, a forward of many tiles and a short K, and a dX of
+    the same leave the short kernels, whose K is dealt to one workgroup's waves only, for the tiles that split it over
+    the chip; layers of ordinary width over few rows stay. The kernels that ran are read from the profile, the results
+    held to fp64 as above (dW's sums run over the rows)."""
+    from laya_amd import ops
+    from laya_amd.device import Context, DeviceArray
+    c = ctx if precision == "fp32" else Context(0)
+    c.set_matmul_precision(precision)
+    r = np.random.default_rng(rows + fan_in)
+    x = r.standard_normal((rows, fan_in)).astype(np.float32)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
+    low = (lambda a: _bf16(a).astype(np.float64)) if precision == "bf16" else (lambda a: a.astype(np.float64))
+    Wp, frozen = ops.Parameter(c, "W", W), ops.Parameter(c, "F", W, False)
+    xd, dyd = DeviceArray.from_numpy(c, x), DeviceArray.from_numpy(c, dy)
+    y, dx = DeviceArray(c, (rows, fan_out)), DeviceArray(c, (rows, fan_in))
+    want_dx, want_dW = low(dy) @ low(W), low(dy).T @ low(x)
+    bar = 1e-6 * max(1.0, np.sqrt(rows / 768))
+
+    got = []
+
+    def run(kind, kernel, call):
+        c.profile_begin()
+        call()
+        if any(k.startswith(kernel) and k.endswith(("_h2s", "_bf16s")) for k in c.profile_end()):
+            got.append(kind)
+
+    run("forward", "gemm_nt", lambda: ops.linear(Wp, None, xd, rows, y))
+    assert _rel(y.numpy(), low(x) @ low(W).T) < 1e-6
+    run("dx", "gemm_nn", lambda: ops.linear_backward(frozen, None, xd, dyd, rows, dx))
+    assert _rel(dx.numpy(), want_dx) < 1e-6
+    run("dw", "gemm_tn", lambda: ops.linear_backward(Wp, None, xd, dyd, rows, None))
+    assert _rel(Wp.gradient_buffer().numpy(), want_dW) < bar
+    Wp.zero_gradient()
+    run("pair", "gemm_bwd_pair", lambda: ops.linear_backward(Wp, None, xd, dyd, rows, dx))
+    assert _rel(dx.numpy(), want_dx) < 1e-6
+    assert _rel(Wp.gradient_buffer().numpy(), want_dW) < bar
+    assert got == short.split()
+    if c is not ctx:
+        c.close()
