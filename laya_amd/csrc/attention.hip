@@ -1715,20 +1715,21 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
         check_launch("attn_dot_kernel");
     }
     {
-        ProfileScope scope(ctx, "attention_bwd_dkv", 2.0 * fb, 0.0);
-        if (a.head_dim == 64)
-            LAYA_LAUNCH(attn_bwd_dkv_kernel<64>, grid, dim3(THREADS), 0, ctx->stream, p);
-        else
-            LAYA_LAUNCH(attn_bwd_dkv_kernel<32>, grid, dim3(THREADS), 0, ctx->stream, p);
-        check_launch("attn_bwd_dkv_kernel");
-    }
-    {
+        // dQ first, as in the other forms: it reads every row's v, which dK/dV overwrites where dqkv is qkv itself.
         ProfileScope scope(ctx, "attention_bwd_dq", 2.0 * fb, 0.0);
         if (a.head_dim == 64)
             LAYA_LAUNCH(attn_bwd_dq_kernel<64>, grid, dim3(THREADS), 0, ctx->stream, p);
         else
             LAYA_LAUNCH(attn_bwd_dq_kernel<32>, grid, dim3(THREADS), 0, ctx->stream, p);
         check_launch("attn_bwd_dq_kernel");
+    }
+    {
+        ProfileScope scope(ctx, "attention_bwd_dkv", 2.0 * fb, 0.0);
+        if (a.head_dim == 64)
+            LAYA_LAUNCH(attn_bwd_dkv_kernel<64>, grid, dim3(THREADS), 0, ctx->stream, p);
+        else
+            LAYA_LAUNCH(attn_bwd_dkv_kernel<32>, grid, dim3(THREADS), 0, ctx->stream, p);
+        check_launch("attn_bwd_dkv_kernel");
     }
 }
 

@@ -221,3 +221,29 @@ def test_short_products_only_where_they_fill_the_chip(ctx, precision, rows, fan_
     assert got == short.split()
     if c is not ctx:
         c.close()
+
+
+@pytest.mark.parametrize("policy", ["fp32", "fp32-split3", "fp32-mfma"])
+@pytest.mark.parametrize("head_dim,lengths,window", [(64, [300, 65], -1), (64, [700, 129], 64), (32, [200, 33], 8)])
+def test_attention_backward_in_place(head_dim, lengths, window, policy):
+    """dqkv may be qkv itself where RoPE is applied to a copy of q and k: v, read from the caller's array, is not
+    overwritten before its last reader is done. The same bits as with an output of its own."""
+    from laya_amd import ops
+    from laya_amd.device import Context, DeviceArray
+    c = Context(0)
+    c.set_matmul_precision(policy)
+    heads, rows = 4, sum(lengths)
+    hidden = heads * head_dim
+    r = np.random.default_rng(rows)
+    qkv = r.standard_normal((rows, 3 * hidden)).astype(np.float32)
+    dctx = DeviceArray.from_numpy(c, r.standard_normal((rows, hidden)).astype(np.float32))
+    segs = ops.Segments(c, np.asarray(lengths, np.int32))
+    shape = ops.AttentionShape(hidden, heads, ops.default_scale(head_dim), window,
+                               ops.Rotary(c, head_dim, 10000.0, max(lengths)), 0.0, 0)
+    q, ctxt, lse = DeviceArray.from_numpy(c, qkv), DeviceArray(c, (rows, hidden)), DeviceArray(c, (rows * heads,))
+    ops.attention_forward(q, segs, shape, ctxt, lse)
+    d = DeviceArray(c, (rows, 3 * hidden))
+    ops.attention_backward(q, segs, shape, dctx, d, ctxt, lse)
+    ops.attention_backward(q, segs, shape, dctx, q, ctxt, lse)
+    np.testing.assert_array_equal(q.numpy(), d.numpy())
+    c.close()
