@@ -369,10 +369,10 @@ int laya_linear_bwd(laya_ctx* ctx, const float* x, const float* dy, int rows, in
         LAYA_REQUIRE(dy && W, "linear_bwd: null tensor");
         LAYA_REQUIRE(!dW || x, "linear_bwd: dW needs x");
         if (dx && dW && db) {
-            // The bias gradient's pass over dy takes dy's magnitude for the pair's two-piece products too.
+            // The bias gradient's pass over dy takes dy's magnitude for the pair's two-piece products too where it can;
+            // else the pair measures it with its other operands, if its kernels need it.
             unsigned* w = operand_ring_word(ctx);
-            column_sum_add(ctx, dy, rows, out, db, w);
-            unsigned char known = 1;
+            unsigned char known = column_sum_add(ctx, dy, rows, out, db, w);
             gemm_backward_pair(ctx, rows, in, out, dy, W, x, dx, nullptr, dW, nullptr, nullptr, AmaxRef{w, &known});
             return;
         }
@@ -685,13 +685,13 @@ int laya_linear_bwd_w(laya_ctx* ctx, const float* x, const float* dy, int rows, 
         LAYA_REQUIRE(dy && W, "linear_bwd: null tensor");
         LAYA_REQUIRE(!dW || x, "linear_bwd: dW needs x");
         LAYA_REQUIRE(!dx_words || dx, "linear_bwd: dx_words without dx");
-        unsigned* w_dy = const_cast<unsigned*>(dy_words);
-        if (db && !w_dy && dx && dW) {  // the bias gradient's pass measures dy for the pair, as laya_linear_bwd does
-            w_dy = operand_ring_word(ctx);
-            column_sum_add(ctx, dy, rows, out, db, w_dy);
+        Given gdy(dy_words);
+        const Given gx(x_words), gw(W_words);
+        if (db && !dy_words && dx && dW) {  // the bias gradient's pass measures dy for the pair, as laya_linear_bwd does
+            gdy.ref = AmaxRef{operand_ring_word(ctx), &gdy.known};
+            gdy.known = column_sum_add(ctx, dy, rows, out, db, gdy.ref.word);
             db = nullptr;
         }
-        const Given gdy(w_dy), gx(x_words), gw(W_words);
         unsigned* wdx = cleared(ctx, dx_words);
         if (dx && dW) {
             gemm_backward_pair(ctx, rows, in, out, dy, W, x, dx, nullptr, dW, nullptr, nullptr, gdy.ref, gw.ref, gx.ref,

@@ -358,9 +358,9 @@ const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, int slot, const float
 void operand_amax_refs(laya_ctx* ctx, AmaxRef ra, const float* a, int rows_a, int cols_a, const unsigned** word_a,
                        AmaxRef rb, const float* b, int rows_b, int cols_b, const unsigned** word_b);
 
-// Σ over rows of a [rows, n] matrix added into out[n], deterministic (bias gradients); amax (optional): max|x|
-// folded into that word group too, in the same pass where the sums take the float4 path.
-void column_sum_add(laya_ctx* ctx, const float* x, int rows, int n, float* out, unsigned* amax = nullptr);
+// Σ over rows of a [rows, n] matrix added into out[n], deterministic (bias gradients); amax (optional): max|x| folded
+// into that word group in the same pass. Returns whether it was: only the float4 path of more than 256 rows does.
+bool column_sum_add(laya_ctx* ctx, const float* x, int rows, int n, float* out, unsigned* amax = nullptr);
 // The context's next operand word group, cleared (the ring operand_amax_ref measures into when the caller keeps
 // no word), for a caller that folds an operand's magnitude into it itself.
 unsigned* operand_ring_word(laya_ctx* ctx);

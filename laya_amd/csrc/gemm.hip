@@ -3602,19 +3602,18 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
     finish_accumulate(ctx, tn, dW_out, in);
 }
 
-void column_sum_add(laya_ctx* ctx, const float* x, int rows, int n, float* out, unsigned* amax) {
-    if (rows <= 0 || n <= 0) return;
+bool column_sum_add(laya_ctx* ctx, const float* x, int rows, int n, float* out, unsigned* amax) {
+    if (rows <= 0 || n <= 0) return false;
     if (n % 4 == 0 && aligned16(x) && aligned16(out) && rows > 256) {
         column_sums(ctx, x, rows, n, nullptr, 1, out, 1, amax);
-        return;
+        return amax != nullptr;
     }
-    if (amax) absmax_into(ctx, x, rows, n, n, amax);
     const int rows_per = 256;
     const int chunks = (rows + rows_per - 1) / rows_per;
     if (chunks <= 1) {
         LAYA_LAUNCH(column_sum_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, x, rows, n, out);
         check_launch("column_sum_kernel");
-        return;
+        return false;
     }
     float* part = static_cast<float*>(ctx->workspace(1, sizeof(float) * (size_t)chunks * n));
     LAYA_LAUNCH(column_partial_kernel, dim3((n + 255) / 256, chunks), dim3(256), 0, ctx->stream, x, rows, n,
@@ -3622,6 +3621,7 @@ void column_sum_add(laya_ctx* ctx, const float* x, int rows, int n, float* out, 
     check_launch("column_partial_kernel");
     LAYA_LAUNCH(column_reduce_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, part, chunks, n, out);
     check_launch("column_reduce_kernel");
+    return false;
 }
 
 }  // namespace laya

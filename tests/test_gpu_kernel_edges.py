@@ -247,3 +247,33 @@ def test_attention_backward_in_place(head_dim, lengths, window, policy):
     ops.attention_backward(q, segs, shape, dctx, q, ctxt, lse)
     np.testing.assert_array_equal(q.numpy(), d.numpy())
     c.close()
+
+
+@pytest.mark.parametrize("words", [False, True])
+@pytest.mark.parametrize("rows,fan_in,fan_out,measured", [(200, 768, 768, 0), (257, 768, 768, 0), (200, 784, 98, 1)])
+def test_biased_backward_measures_only_what_it_reads(ctx, rows, fan_in, fan_out, measured, words):
+    """The bias gradient of few rows is summed without a pass of its own over dY's magnitudes: the short pair reads none,
+    and a pair that the short kernels refuse (a K that is no multiple of 32) measures dY with its other operands, in one
+    launch for each product. The results as without a bias, to the bit."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    r = np.random.default_rng(rows + fan_out)
+    x, W = r.standard_normal((rows, fan_in)).astype(np.float32), r.standard_normal((fan_out, fan_in)).astype(np.float32)
+    dy = r.standard_normal((rows, fan_out)).astype(np.float32)
+    out = []
+    for biased in (False, True):
+        Wp = ops.Parameter(ctx, "W", W)
+        b = ops.Parameter(ctx, "b", np.zeros(fan_out, np.float32)) if biased else None
+        dx = DeviceArray(ctx, (rows, fan_in))
+        dx_words = ops.magnitude_words(ctx) if words else None
+        xd, dyd = DeviceArray.from_numpy(ctx, x), DeviceArray.from_numpy(ctx, dy)
+        ctx.profile_begin()
+        ops.linear_backward(Wp, b, xd, dyd, rows, dx, dx_words=dx_words)
+        launches = ctx.profile_end().get("absmax", {}).get("launches", 0)
+        if biased:
+            assert launches == out[0][2]
+            assert _rel(b.gradient_buffer().numpy(), dy.astype(np.float64).sum(0)) < 1e-6
+        assert (launches > 0) == bool(measured)
+        out.append((dx.numpy(), Wp.gradient_buffer().numpy(), launches))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
