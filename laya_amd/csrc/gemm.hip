@@ -3006,19 +3006,20 @@ double measuring_time(std::initializer_list<std::pair<AmaxRef, double>> operands
 // gemm_short.hip are weighed against: 128 x 128 tiles with K split over idle CUs, the partials written and summed.
 // Fitted to the same shapes as theirs, where it is within 20 % for four in five; the 256-wide tiles that the larger of
 // them take come out near it.
-double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16) {
+// one_piece: a bf16-valued B, taken as one fp16 piece where K is not split.
+double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, bool one_piece = false) {
     const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     GemmParams p{};
     p.K = K;
     const int splits = set_splits(p, fill_splits(ctx, tiles, K, 128));
     const long slots = 2L * ctx->cu_count, rounds = ((long)tiles * splits + slots - 1) / slots;
     const double mb = 4e-6 * M * N;
-    return 7.0 + (bf16 ? 0.75 : 1.3) * rounds * (p.k_per_split / BK) + (splits > 1 ? 0.45 * splits * mb : 0.0) + 0.2 * mb;
+    return 7.0 + (bf16 ? 0.75 : one_piece && splits == 1 ? 1.0 : 1.3) * rounds * (p.k_per_split / BK) + (splits > 1 ? 0.45 * splits * mb : 0.0) + 0.2 * mb;
 }
 
 // The same with the time its operands' magnitudes take (A is M x K and B N x K, however they are stored).
 double product_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, AmaxRef a, AmaxRef b) {
-    return tiles_time(ctx, M, N, K, bf16) + (bf16 ? 0.0 : measuring_time({{a, (double)M * K}, {b, (double)N * K}}));
+    return tiles_time(ctx, M, N, K, bf16, b.bf16) + (bf16 ? 0.0 : measuring_time({{a, (double)M * K}, {b, (double)N * K}}));
 }
 
 }  // namespace

@@ -494,24 +494,32 @@ long chain_of(const ShortGemm& g, int waves) { return ceil_div(ceil_div(g.K, UNI
 
 double megabytes(double floats) { return 4e-6 * floats; }
 
-// Microseconds a product takes here: its rounds of workgroups, each a chain of stages and an epilogue. Work alone does
-// not say it: dW of 768 x 64 over 65,536 rows is twelve workgroups of 256 stages a wave, 460 us here and 130 with K split
-// over the chip; 65536 x 64 -> 768 forward is 12,288 tiles of half a stage a wave, 109 us here and 65 on 256-wide tiles.
-// Fitted to 250 shapes per precision (widths 32 … 4096, 16 … 131,072 rows, back to back on one stream), where it is
-// within 15 % for four in five. Choosing by it and by the other tiles' estimate was within 2 % of the faster of the two
-// in sum over 290 other shapes, forward, dX, dW and pair alike.
+// Memory traffic in MB: A is read by each XCD that has columns of its rows, B once (rows fastest: a tile of B stays on
+// one XCD).
+double traffic_of(const ShortGemm& g, long tiles_n) {
+    return megabytes((double)g.M * g.K * std::min(8L, tiles_n) + (double)g.N * g.K);
+}
+
+// Microseconds a product takes here: its rounds of workgroups, each a chain of stages and an epilogue, and its traffic
+// from the memory-side cache. Work alone does not say it: dW of 768 x 64 over 65,536 rows is twelve workgroups of 256
+// stages a wave, 460 us here and 130 with K split over the chip; 65536 x 64 -> 768 forward is 12,288 tiles of half a
+// stage a wave, 109 us here and 65 on 256-wide tiles. Fitted to 500 shapes (widths 32 … 4096, 16 … 131,072 rows, back to
+// back on one stream), where it is within 10 % for four in five. Choosing by it and by the other tiles' estimate is
+// within 1 % of the faster of the two in sum over 290 other shapes, forward, dX, dW and pair alike.
 double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g) {
-    const bool bf16 = is_bf16(ctx, layout), nt = layout == GemmLayout::NT;
+    const bool bf16 = is_bf16(ctx, layout), accumulate = ep == ShortEpilogue::Accumulate;
     const Shape s = shape_of(ctx, layout, ep, g);
-    const bool small = s.tn == 32;
-    double stage;
-    if (small) stage = bf16 ? 0.34 : 0.87;
-    else if (s.tm == 32) stage = bf16 ? 0.87 : 1.55;
-    else if (s.waves == 4) stage = bf16 ? 1.45 : 2.15;
-    else stage = nt ? (bf16 ? 1.65 : 2.4) : bf16 ? 1.1 : 1.9;
-    const long per_round = (s.waves == 4 || small ? 2L : 1L) * ctx->cu_count;
-    return 2.5 + ceil_div(s.tiles, per_round) * (2.0 + stage * chain_of(g, s.waves)) +
-           (ep == ShortEpilogue::Accumulate ? 0.25 : 0.05) * megabytes((double)g.M * g.N);
+    const long chain = chain_of(g, s.waves), cu = ctx->cu_count;
+    const double out = megabytes((double)g.M * g.N);
+    const double moved = (bf16 ? 0.08 : 0.07) * traffic_of(g, s.tiles / ceil_div(g.M, s.tm));
+    if (s.waves == 4) {  // two workgroups share a CU; the last of an odd number has it to itself
+        const long each = ceil_div(s.tiles, cu);
+        return 2.7 + 0.15 * out + moved + (each / 2) * ((accumulate ? 2.5 : 0.8) + (bf16 ? 1.0 : 1.83) * chain) +
+               (each % 2) * ((accumulate ? 1.8 : 1.3) + (bf16 ? 0.6 : 1.05) * chain);
+    }
+    if (s.tn == 32) return 4.0 + moved + (bf16 ? 0.25 : 0.74) * ceil_div(s.tiles, 2 * cu) * chain;
+    if (s.tm == 32) return 3.6 + moved + (bf16 ? 0.8 : 1.3) * chain;
+    return 4.2 + moved + (accumulate ? 0.15 * out : 0.0) + (bf16 ? 0.95 : 1.7) * ceil_div(s.tiles, cu) * chain;
 }
 
 // As for the forward; and eight waves where dX is few tiles of a long K, which last longest (512 x 768 -> 2304, 96
@@ -520,23 +528,25 @@ int pair_waves(const laya_ctx* ctx, const ShortGemm& nn, long dx_tiles, long dw_
     return dx_tiles + dw_tiles > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048) ? 4 : 8;
 }
 
-// The same of a pair: dX's workgroups, then dW's. Where they come in more than one round the last of dW's begin, on the
-// average, half their length before the others are done.
+// The same of a pair: dX's workgroups, then dW's, of which the last begin, where they come in more than one round, as the
+// others are done.
 double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) {
     const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
     const long dx = tiles_of(nn, ShortEpilogue::Store, 64, 64), dw = tiles_of(tn, ShortEpilogue::Accumulate, 64, 64);
     const int waves = pair_waves(ctx, nn, dx, dw);
     const long slots = (waves == 4 ? 2L : 1L) * ctx->cu_count;
-    const double epilogue = bf16 ? 1.7 : 1.0, stage = bf16 ? (waves == 4 ? 1.3 : 1.15) : waves == 4 ? 1.95 : 1.9;
-    const double a = chain_of(nn, waves) + epilogue, b = chain_of(tn, waves) + epilogue;
+    const double a = chain_of(nn, waves) + 1.0, b = chain_of(tn, waves) + 1.0;  // an epilogue is about a stage
     double span = std::max(a, b);
-    if (dx + dw > slots) span = std::max(span, (dx * a + dw * b) / slots + 0.5 * b);
-    return 4.0 + stage * span;
+    if (dx + dw > slots) span = std::max(span, (dx * a + dw * b) / slots + b);
+    const long tiles_n = ceil_div(nn.N, 64);
+    const double moved = traffic_of(nn, tiles_n) + traffic_of(tn, tiles_n);
+    const double out = megabytes((double)nn.M * nn.N + 2.0 * tn.M * tn.N);
+    if (waves == 4) return 3.1 + (bf16 ? 0.68 : 1.25) * span + 0.075 * moved + 0.14 * out;
+    return 3.4 + (bf16 ? 0.93 : 1.7) * span + 0.06 * moved + 0.07 * out;
 }
 
-// A product runs here only where the estimates differ by more than this; bf16 ones scatter more (3200 x 1152 -> 768, the
-// pair: 50 and 59 estimated, 68 and 56 measured).
-constexpr double MARGIN = 0.95, MARGIN_BF16 = 0.9;
+// A product runs here only where the estimates differ by more than this, about what they scatter by.
+double margin(bool bf16) { return bf16 ? 0.87 : 0.93; }
 
 }  // namespace
 
@@ -545,7 +555,7 @@ bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, c
     const bool bf16 = is_bf16(ctx, layout);
     if (!bf16 && !((ctx->matmul_pair & cls) && (ctx->matmul_split & cls))) return false;
     return work_of(g) <= (bf16 ? FORWARD_LIMIT_BF16 : FORWARD_LIMIT) && short_gemm_fits(g, layout, ep) &&
-           short_time(ctx, layout, ep, g) < (bf16 ? MARGIN_BF16 : MARGIN) * other;
+           short_time(ctx, layout, ep, g) < margin(bf16) * other;
 }
 
 bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, double other) {
@@ -554,7 +564,7 @@ bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& 
     return work_of(nn) <= (bf16 ? PAIR_LIMIT_BF16 : PAIR_LIMIT) &&
            short_gemm_fits(nn, GemmLayout::NN, ShortEpilogue::Store) &&
            short_gemm_fits(tn, GemmLayout::TN, ShortEpilogue::Accumulate) &&
-           pair_time(ctx, nn, tn) < (bf16 ? MARGIN_BF16 : MARGIN) * other;
+           pair_time(ctx, nn, tn) < margin(bf16) * other;
 }
 
 #define SHORT_NP(W, ...)                                                                                   \
