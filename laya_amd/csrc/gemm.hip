@@ -3355,11 +3355,12 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
 }
 
 // The wide pair for split products: dX without residual, dX's K a multiple of 16, dY k-contiguous in
-// float4s. Returns false (nothing launched) when the wide plan does not apply.
+// float4s. Returns false (nothing launched) when the wide plan does not apply, or is an uneven one where `uneven` is
+// not set: launches of their own are faster for a bf16 dX of few tiles (3232 x 1152 -> 768: 56 us and 62).
 // amax_dx (optional): dX's magnitude word group, folded in by the two-piece kernel (*folded set), else
 // left to the caller.
 bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, int in, int out, bool half,
-                        AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx, bool* folded) {
+                        bool uneven, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx, bool* folded) {
     const bool bh = half && nn.B16 && tn.B16;  // W and x from their bf16 copies
     if (out % BKQ != 0 || !operand_fast(nn.A, nn.lda, nn.vec_a, true, nn.M, nn.K)) return false;
     const long lim = 1L << 31;  // buffer offsets of dY, W and x
@@ -3370,7 +3371,7 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
     tn.tiles_n = (in + WT - 1) / WT;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;
     PairPlan s{};
-    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, half, s)) return false;
+    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, half, s) || (s.rest && !uneven)) return false;
     s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * WT * WT));
     const bool pair = !half && (ctx->matmul_pair & 6) == 6;
     if (pair) {
@@ -3435,6 +3436,7 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
                              const __bf16* x16, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx,
                              bool* folded) {
     if (rows == 0) return;
+    bool uneven = true;  // whether the wide pair may leave dW to some of its workers
     {
         ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
         const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
@@ -3446,21 +3448,24 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         PairPlan s{};
         const bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
                                                                (out + WT - 1) / WT * wt_in, rows, bf16, s);
-        double other;
-        if (wide && s.rest)
-            other = 25.0 + 0.75 * std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
-        else if (wide)
+        PairPlan balanced{};  // of 128 x 128 tiles
+        const bool planned =
+            make_pair_plan(ctx, (rows + BM - 1) / BM * t_in, out, (out + BM - 1) / BM * t_in, rows, balanced);
+        double other = (bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
+                       (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16);
+        if (wide && s.rest) {
+            const double rest =
+                25.0 + 0.75 * std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
+            uneven = planned || rest < other;
+            if (uneven) other = rest;
+        } else if (wide) {
             other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
-        else
-            other = (bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
-                    (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16);
+        }
         if (!bf16)
             other += measuring_time({{amax_dy, (double)rows * out}, {amax_W, (double)out * in}, {amax_x, (double)rows * in}});
         // Nor where an fp32 pair runs as exact three-piece splits, the balanced plan below (5600 x 768 -> 768): two
         // pieces would keep rows of dY far below its largest to fewer bits.
-        PairPlan exact{};
-        const bool pieces3 = !bf16 && !wide &&
-                             make_pair_plan(ctx, (rows + BM - 1) / BM * t_in, out, (out + BM - 1) / BM * t_in, rows, exact);
+        const bool pieces3 = !bf16 && !wide && planned;
         if (!pieces3 && short_pair_pays(ctx, nn, tn, other)) {
             short_gemm_pair(ctx, nn, tn);
             *folded = amax_dx != nullptr;
@@ -3481,7 +3486,7 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
     const bool half = (ctx->matmul_bf16 & 6) == 6 && gemm_fits_h(nn, true, false) && gemm_fits_h(tn, false, false);
     tn.mode = ACCUMULATE;
     if ((split || half) &&
-        backward_pair_wide(ctx, nn, tn, rows, in, out, half, amax_dy, amax_W, amax_x, amax_dx, folded))
+        backward_pair_wide(ctx, nn, tn, rows, in, out, half, uneven, amax_dy, amax_W, amax_x, amax_dx, folded))
         return;
     tn.mode = STORE;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;

@@ -132,11 +132,14 @@ def test_short_attention(ctx, lengths, window, p_drop):
 
 
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
-@pytest.mark.parametrize("rows,fan_in,fan_out", [(2500, 3072, 768), (5300, 768, 2304), (6001, 768, 768)])
-def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in, fan_out):
-    """The wide backward pair where a dX tile is more than a worker's share, so that the workers with one more dX tile
-    do no dW: against fp64 on the same operands, 1e-6 relative L2 widened by the square root of K over 768 for dW, whose
-    sums run over the rows."""
+@pytest.mark.parametrize("rows,fan_in,fan_out,bf16_kernel", [
+    (2500, 3072, 768, "gemm_bwd_pair_bf16w"), (6000, 768, 2304, "gemm_bwd_pair_bf16w"),
+    (8003, 768, 2304, "gemm_bwd_pair_bf16w"), (5300, 768, 2304, ""), (6001, 768, 768, ""), (3232, 1152, 768, "gemm_nn_bf16")])
+def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in, fan_out, bf16_kernel):
+    """Pairs whose dX tile is more than a worker's share of the wide plan. In bf16 the workers with one more dX tile do no
+    dW where that pays (the shapes that name the wide kernel: half of the workers busy, and either the balanced plan of
+    128 x 128 tiles would be next or launches of their own are not faster); in fp32 none does. Against fp64 on the same
+    operands, 1e-6 relative L2 widened by the square root of K over 768 for dW, whose sums run over the rows."""
     from laya_amd import ops
     from laya_amd.device import Context, DeviceArray
     c = ctx if precision == "fp32" else Context(0)
@@ -147,11 +150,44 @@ def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in,
     dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
     low = (lambda a: _bf16(a).astype(np.float64)) if precision == "bf16" else (lambda a: a.astype(np.float64))
     Wp, dx = ops.Parameter(c, "W", W), DeviceArray(c, (rows, fan_in))
+    c.profile_begin()
     ops.linear_backward(Wp, None, DeviceArray.from_numpy(c, x), DeviceArray.from_numpy(c, dy), rows, dx)
+    ran = set(c.profile_end())
+    assert not any(k.endswith("_h2w") for k in ran)
+    assert precision == "fp32" or not bf16_kernel or bf16_kernel in ran, ran
     assert _rel(dx.numpy(), low(dy) @ low(W)) < 1e-6
     assert _rel(Wp.gradient_buffer().numpy(), low(dy).T @ low(x)) < 1e-6 * np.sqrt(rows / 768)
     if c is not ctx:
         c.close()
+
+
+def test_uneven_wide_pair_with_a_residual(ctx):
+    """The first layer's QKV backward adds the residual gradient to dX in the wide pair's epilogue; with bf16 products
+    over 8003 tokens some of its workers do no dW. Against the same step's fp32 products at bf16's bar, 2e-2 relative L2
+    (without the residual the embedding gradient would be off by its own size)."""
+    from laya_amd.batch import synthetic_batch
+    from laya_amd.device import Context
+    from laya_amd.model import TrainableDecisionModel
+    mc = mid_config(layers=1)
+    params = random_params(oracle.OracleModel(mc).shapes, 7, std=0.02)
+    lengths = [500] * 15 + [503]
+    batch = synthetic_batch(np.random.default_rng(8), lengths, [4] * 16, [0] * 16, mc.encoder.vocab_size)
+    d = np.random.default_rng(9).standard_normal(batch.n_markers).astype(np.float32)
+    grads = []
+    for policy in ("fp32", "bf16-backward"):
+        c = Context(0)
+        c.set_matmul_precision(policy)
+        m = TrainableDecisionModel(mc, c)
+        m.set_params(params)
+        m.forward(batch, training=False)
+        c.profile_begin()
+        m.backward(d)
+        ran = set(c.profile_end())
+        assert policy == "fp32" or "gemm_bwd_pair_bf16w" in ran
+        grads.append(m.grad("encoder.embeddings.tok_embeddings.weight"))
+        m.close()
+        c.close()
+    assert _rel(grads[1], grads[0].astype(np.float64)) < 2e-2
 
 
 @pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700), (2500, 3072, 768), (8003, 768, 2304),
