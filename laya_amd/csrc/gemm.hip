@@ -2994,19 +2994,10 @@ int fill_splits(const laya_ctx* ctx, int tiles, int K, int min_k) {
     return std::max(1, std::min({slots / tiles, K / min_k, 32}));
 }
 
-// Microseconds that measuring a product's operands adds: one launch over those whose magnitude is not known.
-double measuring_time(std::initializer_list<std::pair<AmaxRef, double>> operands) {
-    double bytes = 0.0;
-    for (const auto& [ref, elements] : operands)
-        if (!ref.word || !*ref.known) bytes += 4.0 * elements;
-    return bytes > 0.0 ? 3.3 + 0.14e-6 * bytes : 0.0;
-}
-
-// Microseconds a product takes on the tiles of this file, its operands' magnitudes known, as the short products of
-// gemm_short.hip are weighed against: 128 x 128 tiles with K split over idle CUs, the partials written and summed.
-// Fitted to the same shapes as theirs, where it is within 20 % for four in five; the 256-wide tiles that the larger of
-// them take come out near it.
-// one_piece: a bf16-valued B, taken as one fp16 piece where K is not split.
+// Microseconds a product takes on the tiles of this file, as the short products of gemm_short.hip are weighed against:
+// 128 x 128 tiles with K split over idle CUs, the partials written and summed. Fitted to the same shapes as theirs, where
+// it is within 20 % for four in five; the 256-wide tiles that the larger of them take come out near it. one_piece: a
+// bf16-valued B, taken as one fp16 piece where K is not split.
 double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, bool one_piece = false) {
     const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     GemmParams p{};
@@ -3014,12 +3005,18 @@ double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, bool one_
     const int splits = set_splits(p, fill_splits(ctx, tiles, K, 128));
     const long slots = 2L * ctx->cu_count, rounds = ((long)tiles * splits + slots - 1) / slots;
     const double mb = 4e-6 * M * N;
-    return 7.0 + (bf16 ? 0.75 : one_piece && splits == 1 ? 1.0 : 1.3) * rounds * (p.k_per_split / BK) + (splits > 1 ? 0.45 * splits * mb : 0.0) + 0.2 * mb;
+    const double stage = bf16 ? 0.75 : one_piece && splits == 1 ? 1.0 : 1.3;
+    return 7.0 + stage * rounds * (p.k_per_split / BK) + (splits > 1 ? 0.45 * splits : 0.0) * mb + 0.2 * mb;
 }
 
-// The same with the time its operands' magnitudes take (A is M x K and B N x K, however they are stored).
-double product_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, AmaxRef a, AmaxRef b) {
-    return tiles_time(ctx, M, N, K, bf16, b.bf16) + (bf16 ? 0.0 : measuring_time({{a, (double)M * K}, {b, (double)N * K}}));
+// What to count of measuring an fp32 product's operands, 3.3 us and 0.14 per MB where their magnitudes are not known: half
+// of it whether they are known or not, so that a caller who keeps them gets the same bits as one who does not. Over 3,300
+// products that costs the one 1 % and the other 3 % of the time that choosing by what is known would give.
+double measuring_time(bool bf16, double elements) { return bf16 ? 0.0 : 0.5 * (3.3 + 0.14 * 4e-6 * elements); }
+
+// A product's time with that: A is M x K and B N x K, however they are stored.
+double product_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, bool one_piece) {
+    return tiles_time(ctx, M, N, K, bf16, one_piece) + measuring_time(bf16, ((double)M + N) * K);
 }
 
 }  // namespace
@@ -3061,7 +3058,7 @@ void gemm(laya_ctx* ctx, GemmLayout layout, GemmEpilogue ep, int M, int N, int K
         const ShortEpilogue se =
             ep == GemmEpilogue::Store ? ShortEpilogue::Store : ShortEpilogue::Accumulate;
         const int cls = layout == GemmLayout::NT ? 1 : layout == GemmLayout::NN ? 2 : 4;
-        if (short_gemm_pays(ctx, layout, se, g, product_time(ctx, M, N, K, ctx->matmul_bf16 & cls, amax_a, amax_b))) {
+        if (short_gemm_pays(ctx, layout, se, g, product_time(ctx, M, N, K, ctx->matmul_bf16 & cls, amax_b.bf16))) {
             short_gemm(ctx, layout, se, g);
             return;
         }
@@ -3152,7 +3149,7 @@ void gemm_rope(laya_ctx* ctx, int M, int N, int K, const float* A, const float* 
     g.rope_cos = cos_t;
     g.rope_sin = sin_t;
     g.rope_cols = rope_cols;
-    const double tiles_us = product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_a, amax_b);
+    const double tiles_us = product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_b.bf16);
     if (rope_cols <= N && pos && cos_t && sin_t &&
         short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Rope, g, tiles_us)) {
         short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Rope, g);
@@ -3256,7 +3253,7 @@ void gemm_geglu(laya_ctx* ctx, int M, int inter, int K, const float* x, const fl
     // Against the product and a GeGLU pass over its output (12 bytes a value of act, at 5 TB/s).
     const double geglu_us = 4.0 + 0.2 * 12e-6 * M * inter;
     if (short_gemm_pays(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g,
-                        product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_x, amax_W) + geglu_us)) {
+                        product_time(ctx, M, N, K, ctx->matmul_bf16 & 1, amax_W.bf16) + geglu_us)) {
         short_gemm(ctx, GemmLayout::NT, ShortEpilogue::Geglu, g);
         return;
     }
@@ -3461,8 +3458,7 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         } else if (wide) {
             other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
         }
-        if (!bf16)
-            other += measuring_time({{amax_dy, (double)rows * out}, {amax_W, (double)out * in}, {amax_x, (double)rows * in}});
+        other += measuring_time(bf16, (double)rows * out + (double)out * in + (double)rows * in);
         // Nor where an fp32 pair runs as exact three-piece splits, the balanced plan below (5600 x 768 -> 768): two
         // pieces would keep rows of dY far below its largest to fewer bits.
         const bool pieces3 = !bf16 && !wide && planned;

@@ -546,7 +546,7 @@ double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) 
 }
 
 // A product runs here only where the estimates differ by more than this, about what they scatter by.
-double margin(bool bf16) { return bf16 ? 0.87 : 0.93; }
+double margin(bool bf16) { return bf16 ? 0.87 : 0.95; }
 
 }  // namespace
 

@@ -313,3 +313,33 @@ def test_biased_backward_measures_only_what_it_reads(ctx, rows, fan_in, fan_out,
         out.append((dx.numpy(), Wp.gradient_buffer().numpy(), launches))
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("rows,fan_in,fan_out", [(1100, 768, 2304), (1618, 2624, 1024), (1618, 768, 3072),
+                                                 (2200, 768, 2304), (2200, 1152, 768), (2700, 1024, 1024),
+                                                 (3200, 1152, 768), (4800, 768, 768), (8192, 768, 32)])
+def test_known_magnitudes_change_no_bits(ctx, rows, fan_in, fan_out):
+    """Where the short products and the other tiles take about as long, the choice is the same whether the caller keeps
+    the operands' magnitude words (and so spares their measuring) or not: the same bits."""
+    from laya_amd import ops
+    from laya_amd._native import check, lib
+    from laya_amd.device import DeviceArray
+    r = np.random.default_rng(rows)
+    x, W, dy = (DeviceArray.from_numpy(ctx, r.standard_normal(s).astype(np.float32))
+                for s in ((rows, fan_in), (fan_out, fan_in), (rows, fan_out)))
+    xw, ww, dyw = (ops.magnitude_words(ctx) for _ in range(3))
+    for a, w in ((x, xw), (W, ww), (dy, dyw)):
+        ops.measure_words(ctx, a, w)
+    runs = []
+    for words in ((None, None, None), (xw.ptr, ww.ptr, dyw.ptr)):
+        y, dx, dW = (DeviceArray(ctx, s) for s in ((rows, fan_out), (rows, fan_in), (fan_out, fan_in)))
+        one_dx, one_dW = DeviceArray(ctx, (rows, fan_in)), DeviceArray(ctx, (fan_out, fan_in))
+        size = (rows, fan_in, fan_out)
+        check(lib().laya_linear_fwd_w(ctx.handle, x.ptr, *size[:2], W.ptr, fan_out, None, None, y.ptr, words[0], words[1],
+                                      None))
+        for d, g in ((dx, dW), (one_dx, None), (None, one_dW)):
+            check(lib().laya_linear_bwd_w(ctx.handle, x.ptr, dy.ptr, *size, W.ptr, d and d.ptr, g and g.ptr, None,
+                                          words[0], words[2], words[1], None))
+        runs.append([a.numpy() for a in (y, dx, dW, one_dx, one_dW)])
+    for a, b in zip(*runs):
+        np.testing.assert_array_equal(a, b)
