@@ -3457,13 +3457,13 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
             if (uneven) other = rest;
         } else if (wide) {
             other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
+        } else if (planned && !bf16) {
+            other = 55.0 + 2.15 * balanced.W / balanced.G;
         }
         other += measuring_time(bf16, (double)rows * out + (double)out * in + (double)rows * in);
-        // Nor where an fp32 pair runs as exact three-piece splits, the balanced plan below (5600 x 768 -> 768): two
-        // pieces would keep rows of dY far below its largest to fewer bits.
-        const bool pieces3 = !bf16 && !wide && planned;
-        if (!pieces3 && short_pair_pays(ctx, nn, tn, other)) {
-            short_gemm_pair(ctx, nn, tn);
+        const bool lines = !bf16 && !wide && planned;  // exact three-piece splits would follow
+        if (short_pair_pays(ctx, nn, tn, lines, other)) {
+            short_gemm_pair(ctx, nn, tn, lines);
             *folded = amax_dx != nullptr;
             return;
         }

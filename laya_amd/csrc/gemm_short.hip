@@ -171,6 +171,55 @@ __device__ __forceinline__ int wave_scale_exp(const float (&v)[I][2][8]) {
     return pair_scale_exp(u);
 }
 
+// Scales of a line (a row of A, a column of B) of its own rather than of the wave's tile: each lane holds 16 of its
+// line's 32 values, the lane 32 away the rest. e: the lines' exponents; lowered where a value would leave fp16's range,
+// with two bits to spare (a line's later values seldom reach four times its first 32's largest; below, the low piece's
+// floor is still 2^-37 of the line's largest). drop: how far; whether any line's was, in the whole wave.
+constexpr int NO_SCALE = 200;  // before a line's first stage
+template <int I>
+__device__ __forceinline__ bool line_scale_exps(const float (&v)[I][2][8], int (&e)[I], int (&drop)[I]) {
+    auto both = [](unsigned u) {
+#ifdef __HIP_DEVICE_COMPILE__
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return max((unsigned)r[0], (unsigned)r[1]);
+#else
+        return u;
+#endif
+    };
+    unsigned u[I], top = 0;
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+        float m = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int k = 0; k < 8; k += 2) m = max3_abs(m, v[i][s][k], v[i][s][k + 1]);
+        u[i] = both(__builtin_bit_cast(unsigned, m));
+        top = max(top, u[i]);
+    }
+    if (__any(top >= 0x7f800000u)) {  // an infinity or NaN among them: the largest finite ones, value by value
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+            unsigned f = 0;
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) f = max(f, amax_bits(v[i][s][k]));
+            u[i] = both(f);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+        const int p = pair_scale_exp(u[i]), n = e[i] > p ? p - 2 : e[i];
+        drop[i] = n - e[i];
+        e[i] = n;
+    }
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < I; ++i) any |= drop[i];
+    return __any(any);
+}
+
 template <int NP>
 struct Frag {
     f16x8 hi, lo;
@@ -209,7 +258,8 @@ constexpr int wave_floats() {
 
 // One output tile by one workgroup of W waves. AK / BK: A / B contiguous along K (K a multiple of 32 then). EP: the
 // epilogue; N and the leading dimensions of C and R multiples of 4, their bases 16-byte aligned. smem: W · wave_floats.
-template <bool AK, bool BK, int TM, int TN, ShortEpilogue EP, int W, int NP>
+// LINES: two-piece scales by row of A and column of B instead of by wave, which keep lines far below the tile's largest.
+template <bool AK, bool BK, int TM, int TN, ShortEpilogue EP, int W, int NP, bool LINES = false>
 __device__ __forceinline__ void short_tile(const ShortGemm& p, int tile, float* smem) {
     constexpr int I = TM / 32, J = TN / 32, THREADS = 64 * W;
     constexpr int STAGE = UNIT * (TM + TN);
@@ -229,7 +279,18 @@ __device__ __forceinline__ void short_tile(const ShortGemm& p, int tile, float* 
             for (int j = 0; j < J; ++j) f(acc[i][j], sum[i][j]);
     };
     each([](f32x16& a, f32x16& t) { a = t = f32x16{}; });
-    int ea = 126, eb = 126;
+    static_assert(!LINES || NP == 2, "bf16 products have no scales");
+    int ea = 126, eb = 126, la[I], lb[J];
+#pragma unroll
+    for (int i = 0; i < I; ++i) la[i] = NO_SCALE;
+#pragma unroll
+    for (int j = 0; j < J; ++j) lb[j] = NO_SCALE;
+    auto rescale = [&](int i, int j, int r, int d) {
+        acc[i][j][r] = __builtin_amdgcn_ldexpf(acc[i][j][r], d);
+        sum[i][j][r] = __builtin_amdgcn_ldexpf(sum[i][j][r], d);
+    };
+    // A value of the lane that holds row 8·(r / 4) + 4h + r mod 4 of A's group, that of accumulator register r.
+    auto of_row = [&](int x, int r) { return __builtin_amdgcn_ds_bpermute(4 * (8 * (r >> 2) + 4 * h + (r & 3)), x); };
     {
         float* stage = smem + w * STAGE;
         std::conditional_t<AK, SideK<TM>, SideMN> a(p.A, p.lda, p.M, p.K, m0, lane, stage, 0);
@@ -256,12 +317,25 @@ __device__ __forceinline__ void short_tile(const ShortGemm& p, int tile, float* 
             {
                 float v[I][2][8];
                 a.fetch(v, lr, h);
-                if constexpr (NP == 2) na = min(ea, wave_scale_exp(v));
-                const float sc = exp2_int(na);
+                if constexpr (LINES) {
+                    int d[I];
+                    if (line_scale_exps(v, la, d) && u > ub) {
+#pragma unroll
+                        for (int i = 0; i < I; ++i)
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) {
+                                const int dr = of_row(d[i], r);
+#pragma unroll
+                                for (int j = 0; j < J; ++j) rescale(i, j, r, dr);
+                            }
+                    }
+                } else if constexpr (NP == 2) {
+                    na = min(ea, wave_scale_exp(v));
+                }
 #pragma unroll
                 for (int i = 0; i < I; ++i)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) fa[i][s].set(v[i][s], sc);
+                    for (int s = 0; s < 2; ++s) fa[i][s].set(v[i][s], exp2_int(LINES ? la[i] : na));
             }
             __builtin_amdgcn_sched_barrier(0);
             {
@@ -272,14 +346,25 @@ __device__ __forceinline__ void short_tile(const ShortGemm& p, int tile, float* 
                     a.issue((u + 1) * UNIT);
                     b.issue((u + 1) * UNIT);
                 }
-                if constexpr (NP == 2) nb = min(eb, wave_scale_exp(v));
-                const float sc = exp2_int(nb);
+                if constexpr (LINES) {
+                    int d[J];
+                    if (line_scale_exps(v, lb, d) && u > ub) {
+#pragma unroll
+                        for (int j = 0; j < J; ++j)
+#pragma unroll
+                            for (int i = 0; i < I; ++i)
+#pragma unroll
+                                for (int r = 0; r < 16; ++r) rescale(i, j, r, d[j]);
+                    }
+                } else if constexpr (NP == 2) {
+                    nb = min(eb, wave_scale_exp(v));
+                }
 #pragma unroll
                 for (int j = 0; j < J; ++j)
 #pragma unroll
-                    for (int s = 0; s < 2; ++s) fb[j][s].set(v[j][s], sc);
+                    for (int s = 0; s < 2; ++s) fb[j][s].set(v[j][s], exp2_int(LINES ? lb[j] : nb));
             }
-            if constexpr (NP == 2) {
+            if constexpr (NP == 2 && !LINES) {
                 const int d = na + nb - ea - eb;
                 if (d < 0 && u > ub)
                     each([&](f32x16& a, f32x16& t) {
@@ -317,10 +402,11 @@ __device__ __forceinline__ void short_tile(const ShortGemm& p, int tile, float* 
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int q = 8 * (r >> 2) + 4 * h + (r & 3), row = AK ? 32 * i + q : I * q + i;
+                const int er = LINES ? of_row(la[i], r) : 0;
                 float v[J];
 #pragma unroll
                 for (int j = 0; j < J; ++j)
-                    v[j] = NP == 2 ? __builtin_amdgcn_ldexpf(acc[i][j][r], ex) : acc[i][j][r];
+                    v[j] = NP == 2 ? __builtin_amdgcn_ldexpf(acc[i][j][r], LINES ? -(er + lb[j]) : ex) : acc[i][j][r];
                 if constexpr (BK) {
 #pragma unroll
                     for (int j = 0; j < J; ++j) red[row * TN + 32 * j + lr] = v[j];
@@ -417,15 +503,18 @@ __global__ __launch_bounds__(64 * W, 2) void short_gemm_kernel(ShortGemm p) {
     short_tile<AK, BK, TM, TN, EP, W, NP>(p, xcd_tile(blockIdx.x, gridDim.x), smem);
 }
 
-// dX's tiles, then dW's, each over all XCDs: neither product reads what the other writes.
-template <int W, int NP>
+// dX's tiles, then dW's, each over all XCDs: neither product reads what the other writes. LINES costs 6 to 12 % (512 x
+// 768 -> 2304 27 us and 31; 256 registers and ten spilled to the rescaling) and is for pairs that would run as exact
+// three-piece splits otherwise: 1618 x 2624 -> 1024 139 us there, 100 here, the worst row or column of dX and dW off by
+// 1.6e-7 where rows or columns lie 2^-26 below the others, and by 4e-7 there.
+template <int W, int NP, bool LINES>
 __global__ __launch_bounds__(64 * W, 2) void short_pair_kernel(ShortGemm nn, ShortGemm tn, int dx_tiles) {
     __shared__ __attribute__((aligned(16))) float smem[W * 64 * 64];
     const int block = blockIdx.x;
     if (block < dx_tiles)
-        short_tile<true, false, 64, 64, ShortEpilogue::Store, W, NP>(nn, xcd_tile(block, dx_tiles), smem);
+        short_tile<true, false, 64, 64, ShortEpilogue::Store, W, NP, LINES>(nn, xcd_tile(block, dx_tiles), smem);
     else
-        short_tile<false, false, 64, 64, ShortEpilogue::Accumulate, W, NP>(
+        short_tile<false, false, 64, 64, ShortEpilogue::Accumulate, W, NP, LINES>(
             tn, xcd_tile(block - dx_tiles, gridDim.x - dx_tiles), smem);
 }
 
@@ -459,7 +548,7 @@ bool short_gemm_fits(const ShortGemm& g, GemmLayout layout, ShortEpilogue ep) {
 }
 
 // Up to how many multiply-adds a product may run here: the range over which the times below were fitted.
-constexpr double FORWARD_LIMIT = 4.0e9, FORWARD_LIMIT_BF16 = 2.0e9, PAIR_LIMIT = 5.0e9, PAIR_LIMIT_BF16 = 3.0e9;
+constexpr double FORWARD_LIMIT = 4.0e9, FORWARD_LIMIT_BF16 = 2.0e9, PAIR_LIMIT = 5.0e9, PAIR_LIMIT_BF16 = 3.0e9, PAIR_LIMIT_LINES = 9.0e9;
 
 double work_of(const ShortGemm& g) { return (double)g.M * g.N * g.K; }
 
@@ -524,16 +613,17 @@ double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, cons
 
 // As for the forward; and eight waves where dX is few tiles of a long K, which last longest (512 x 768 -> 2304, 96
 // tiles: 27 us with eight waves, 32 with four; 800 rows, 156 tiles: 41 and 36).
-int pair_waves(const laya_ctx* ctx, const ShortGemm& nn, long dx_tiles, long dw_tiles) {
-    return dx_tiles + dw_tiles > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048) ? 4 : 8;
+// Pairs scaled by line have at least 400 tiles: the balanced plan whose place they take needs 100 of 128 x 128 for dX.
+int pair_waves(const laya_ctx* ctx, const ShortGemm& nn, long dx_tiles, long dw_tiles, bool lines) {
+    return lines || (dx_tiles + dw_tiles > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048)) ? 4 : 8;
 }
 
 // The same of a pair: dX's workgroups, then dW's, of which the last begin, where they come in more than one round, as the
 // others are done.
-double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) {
+double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, bool lines) {
     const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
     const long dx = tiles_of(nn, ShortEpilogue::Store, 64, 64), dw = tiles_of(tn, ShortEpilogue::Accumulate, 64, 64);
-    const int waves = pair_waves(ctx, nn, dx, dw);
+    const int waves = pair_waves(ctx, nn, dx, dw, lines);
     const long slots = (waves == 4 ? 2L : 1L) * ctx->cu_count;
     const double a = chain_of(nn, waves) + 1.0, b = chain_of(tn, waves) + 1.0;  // an epilogue is about a stage
     double span = std::max(a, b);
@@ -541,7 +631,7 @@ double pair_time(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn) 
     const long tiles_n = ceil_div(nn.N, 64);
     const double moved = traffic_of(nn, tiles_n) + traffic_of(tn, tiles_n);
     const double out = megabytes((double)nn.M * nn.N + 2.0 * tn.M * tn.N);
-    if (waves == 4) return 3.1 + (bf16 ? 0.68 : 1.25) * span + 0.075 * moved + 0.14 * out;
+    if (waves == 4) return 3.1 + (bf16 ? 0.68 : lines ? 1.35 : 1.25) * span + 0.075 * moved + 0.14 * out;
     return 3.4 + (bf16 ? 0.93 : 1.7) * span + 0.06 * moved + 0.07 * out;
 }
 
@@ -558,13 +648,13 @@ bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, c
            short_time(ctx, layout, ep, g) < margin(bf16) * other;
 }
 
-bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, double other) {
+bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, bool lines, double other) {
     const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
     if (!bf16 && ((ctx->matmul_bf16 & 6) || (ctx->matmul_pair & 6) != 6 || (ctx->matmul_split & 6) != 6)) return false;
-    return work_of(nn) <= (bf16 ? PAIR_LIMIT_BF16 : PAIR_LIMIT) &&
+    return work_of(nn) <= (bf16 ? PAIR_LIMIT_BF16 : lines ? PAIR_LIMIT_LINES : PAIR_LIMIT) &&
            short_gemm_fits(nn, GemmLayout::NN, ShortEpilogue::Store) &&
            short_gemm_fits(tn, GemmLayout::TN, ShortEpilogue::Accumulate) &&
-           pair_time(ctx, nn, tn) < margin(bf16) * other;
+           pair_time(ctx, nn, tn, lines) < margin(bf16) * other;
 }
 
 #define SHORT_NP(W, ...)                                                                                   \
@@ -612,20 +702,21 @@ void short_gemm(laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, ShortGemm g)
 }
 #undef SHORT_NP
 
-void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn) {
+void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn, bool lines) {
     const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
     set_tiles(nn, ShortEpilogue::Store, 64, 64);
     set_tiles(tn, ShortEpilogue::Accumulate, 64, 64);
     const int dx_tiles = nn.tiles_m * nn.tiles_n;
     const dim3 grid(dx_tiles + tn.tiles_m * tn.tiles_n);
-    const bool w4 = pair_waves(ctx, nn, dx_tiles, (long)grid.x - dx_tiles) == 4;
+    const bool w4 = pair_waves(ctx, nn, dx_tiles, (long)grid.x - dx_tiles, lines) == 4;
     ProfileScope scope(ctx, bf16 ? "gemm_bwd_pair_bf16s" : "gemm_bwd_pair_h2s", 4.0 * nn.M * nn.N * (double)nn.K, 0.0);
-#define SHORT_PAIR(W, NP) \
-    LAYA_LAUNCH((short_pair_kernel<W, NP>), grid, dim3(64 * W), 0, ctx->stream, nn, tn, dx_tiles)
-    if (bf16 && w4) SHORT_PAIR(4, 1);
-    else if (bf16) SHORT_PAIR(8, 1);
-    else if (w4) SHORT_PAIR(4, 2);
-    else SHORT_PAIR(8, 2);
+#define SHORT_PAIR(...) \
+    LAYA_LAUNCH((short_pair_kernel<__VA_ARGS__>), grid, dim3(w4 ? 256 : 512), 0, ctx->stream, nn, tn, dx_tiles)
+    if (bf16 && w4) SHORT_PAIR(4, 1, false);
+    else if (bf16) SHORT_PAIR(8, 1, false);
+    else if (lines) SHORT_PAIR(4, 2, true);
+    else if (w4) SHORT_PAIR(4, 2, false);
+    else SHORT_PAIR(8, 2, false);
 #undef SHORT_PAIR
     check_launch("short_pair_kernel");
 }

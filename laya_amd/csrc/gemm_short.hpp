@@ -30,8 +30,9 @@ struct ShortGemm {
 // operands): its shape allows it and these tiles take less time than `other`, gemm.hip's in microseconds.
 bool short_gemm_pays(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g, double other);
 void short_gemm(laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, ShortGemm g);
-// A linear layer's dX (NN, Store) and dW (TN, Accumulate) in one launch.
-bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, double other);
-void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn);
+// A linear layer's dX (NN, Store) and dW (TN, Accumulate) in one launch. lines: fp32 operands scaled by row and column,
+// for pairs that exact three-piece splits would compute otherwise.
+bool short_pair_pays(const laya_ctx* ctx, const ShortGemm& nn, const ShortGemm& tn, bool lines, double other);
+void short_gemm_pair(laya_ctx* ctx, ShortGemm nn, ShortGemm tn, bool lines);
 
 }  // namespace laya

@@ -190,26 +190,62 @@ def test_uneven_wide_pair_with_a_residual(ctx):
     assert _rel(grads[1], grads[0].astype(np.float64)) < 2e-2
 
 
-@pytest.mark.parametrize("rows,fan_in,fan_out", [(12345, 768, 700), (2500, 3072, 768), (8003, 768, 2304),
-                                                 (1400, 3072, 768), (5600, 768, 768), (1600, 2624, 1024)])
-def test_backward_pairs_on_exact_splits_keep_small_rows(ctx, rows, fan_in, fan_out):
-    """fp32 backward pairs that run as exact three-piece splits: dY rows 2^-26 below the rest, each of which a two-piece
-    product under a scale of the others would keep to about 2^(26-39) = 1e-4, come out to fp32 precision (a sum of K
-    terms rounded 2^-24 each: 2e-6 holds K = 2304)."""
+@pytest.mark.parametrize("rows,fan_in,fan_out,kernel", [
+    (12345, 768, 700, "x6"), (8003, 768, 2304, "x6"), (5600, 768, 768, "x6"), (2500, 3072, 768, "h2s"),
+    (1400, 3072, 768, "h2s"), (1403, 3076, 800, "h2s"), (1600, 2624, 1024, "h2s")])
+def test_backward_pairs_keep_lines_far_below_the_largest(ctx, rows, fan_in, fan_out, kernel):
+    """fp32 backward pairs on exact three-piece splits, or on two pieces scaled by row and column: rows and columns of dY,
+    columns of W and of x 2^-26 below the rest, each of which a two-piece product under a scale of the others would keep
+    to about 2^(26-39) = 1e-4, come out to fp32 precision, row by row and column by column (a sum of K terms rounded 2^-24
+    each: 2e-6 holds dX's K of up to 2304, widened by the square root of the rows over 2304 for dW's)."""
     from laya_amd import ops
     from laya_amd.device import DeviceArray
     r = np.random.default_rng(rows + fan_out)
     x = r.standard_normal((rows, fan_in)).astype(np.float32)
     W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
     dy = (1e-4 * r.standard_normal((rows, fan_out))).astype(np.float32)
-    dy[7::50] *= np.float32(2.0 ** -26)
+    tiny = np.float32(2.0 ** -26)
+    dy[7::50] *= tiny
+    dy[:, 5::40] *= tiny
+    W[:, 3::60] *= tiny
+    x[:, 11::30] *= tiny
     Wp, dx = ops.Parameter(ctx, "W", W), DeviceArray(ctx, (rows, fan_in))
     ctx.profile_begin()
     ops.linear_backward(Wp, None, DeviceArray.from_numpy(ctx, x), DeviceArray.from_numpy(ctx, dy), rows, dx)
-    assert "gemm_bwd_pair_x6" in ctx.profile_end()
-    want = dy.astype(np.float64) @ W.astype(np.float64)
-    assert (np.linalg.norm(dx.numpy() - want, axis=1) / np.linalg.norm(want, axis=1)).max() < 2e-6
-    assert _rel(Wp.gradient_buffer().numpy(), dy.astype(np.float64).T @ x.astype(np.float64)) < 1e-6 * np.sqrt(rows / 768)
+    assert "gemm_bwd_pair_" + kernel in ctx.profile_end()
+    dy64, W64, x64 = (a.astype(np.float64) for a in (dy, W, x))
+    bar = 2e-6 * max(1.0, np.sqrt(rows / 2304))
+    for got, want, limit in ((dx.numpy(), dy64 @ W64, 2e-6), (Wp.gradient_buffer().numpy(), dy64.T @ x64, bar)):
+        for axis in (0, 1):
+            e = np.linalg.norm(got - want, axis=axis) / np.linalg.norm(want, axis=axis)
+            print(rows, fan_in, fan_out, kernel, "worst line", e.max())
+            assert e.max() < limit
+
+
+def test_backward_pair_scaled_by_line_with_non_finite_operands(ctx):
+    """A NaN or an infinity in dY stays in its own row of dX and its own row of dW; the scales of its lines come from
+    their finite values. The other lines are held to fp64 as above. Rows of dY grow by 2^20 on the way down, so that the
+    scales of dW's lines are lowered again and again."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    rows, fan_in, fan_out = 1403, 3076, 800
+    r = np.random.default_rng(4)
+    x = r.standard_normal((rows, fan_in)).astype(np.float32)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    dy = (r.standard_normal((rows, fan_out)) * 2.0 ** np.linspace(-30, -10, rows)[:, None]).astype(np.float32)
+    clean = dy.copy()
+    dy[700, 41], dy[90, 300], clean[700, 41], clean[90, 300] = np.inf, np.nan, 0.0, 0.0
+    Wp, dxd = ops.Parameter(ctx, "W", W), DeviceArray(ctx, (rows, fan_in))
+    ctx.profile_begin()
+    ops.linear_backward(Wp, None, DeviceArray.from_numpy(ctx, x), DeviceArray.from_numpy(ctx, dy), rows, dxd)
+    assert "gemm_bwd_pair_h2s" in ctx.profile_end()
+    dx, dW = dxd.numpy(), Wp.gradient_buffer().numpy()
+    for got, want, bad in ((dx, clean.astype(np.float64) @ W.astype(np.float64), (700, 90)),
+                           (dW, clean.astype(np.float64).T @ x.astype(np.float64), (41, 300))):
+        lines = np.isin(np.arange(len(got)), bad)
+        assert not np.isfinite(got[lines]).any()
+        e = np.linalg.norm(got[~lines] - want[~lines], axis=1) / np.linalg.norm(want[~lines], axis=1)
+        assert e.max() < 2e-6
 
 
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
