@@ -41,7 +41,10 @@ def dev(ctx, a):
                                           (4100, 64, 96), (9000, 768, 2304),
                                           # the backward pair on 256 x 256 tiles (ragged columns, ragged last
                                           # dW unit; the model's shapes)
-                                          (11000, 1148, 768), (13871, 768, 2304)])
+                                          (11000, 1148, 768), (13871, 768, 2304),
+                                          # the balanced pair of 128 x 128 tiles: widths that the wide one refuses,
+                                          # dY in float4s and not
+                                          (9000, 768, 2300), (9000, 768, 2302)])
 def test_bf16_linear_is_the_product_of_rounded_operands(ctx, rows, inn, out):
     """Forward with bias and residual (NT), dx (NN) and dW accumulated twice (TN, split-K at 4100 and 9000
     rows), in bf16."""

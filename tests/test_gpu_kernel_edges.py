@@ -103,7 +103,8 @@ def test_short_product_with_non_finite_operands(ctx):
 
 @pytest.mark.parametrize("p_drop", [0.0, 0.2])
 @pytest.mark.parametrize("window", [-1, 64])
-@pytest.mark.parametrize("lengths", [[1], [31, 33, 1], [128], [129, 32], [189], [300, 7], [640], [513, 512]])
+@pytest.mark.parametrize("lengths", [[1], [31, 33, 1], [128], [129, 32], [189], [300, 7], [640], [513, 512],
+                                     [1000], [513, 300]])
 def test_short_attention(ctx, lengths, window, p_drop):
     """Attention of grids small enough for 32 rows to a workgroup (up to 64 workgroups of 128 rows; 96 without a window
     on segments of 512 and more), where each wave takes a subtile of 32 keys or queries, and the next larger grids: row
@@ -379,3 +380,68 @@ def test_known_magnitudes_change_no_bits(ctx, rows, fan_in, fan_out):
         runs.append([a.numpy() for a in (y, dx, dW, one_dx, one_dW)])
     for a, b in zip(*runs):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("lengths", [(33, 20), (64,), (129, 61), (404,)])
+@pytest.mark.parametrize("inter", [1140, 1152])
+def test_short_rope_and_geglu_epilogues(ctx, lengths, inter):
+    """The QKV projection's RoPE and the MLP's GeGLU in the short products' epilogues: rows on both sides of a tile's edge
+    and a GeGLU width that is no multiple of a tile's 32 columns, against the fp64 oracle (logits to 1e-5, as at the
+    other widths); and their bf16 copies, which bf16 backward products read: the gradients with the copies are those
+    without, to the bit."""
+    from helpers import mixed_batch
+    from laya_amd.device import Context
+    from laya_amd.model import TrainableDecisionModel
+    mc = mid_config(layers=2, inter=inter)
+    o = oracle.OracleModel(mc, double=True)
+    params = random_params(o.shapes, 11, std=0.03)
+    batch = mixed_batch(np.random.default_rng(12), list(lengths), mc.encoder.vocab_size)
+    o.set_params(params)
+    want = o.forward(batch, training=False)
+    m = TrainableDecisionModel(mc, ctx)
+    m.set_params(params)
+    ctx.profile_begin()
+    got = m.forward(batch, training=False)
+    ran = set(ctx.profile_end())
+    assert "gemm_nt_h2s" in ran and "geglu_fwd" not in ran
+    assert _rel(got, want) < 1e-5
+    m.close()
+    d = np.random.default_rng(13).standard_normal(batch.n_markers).astype(np.float32)
+    grads = []
+    for copies in (True, False):
+        c = Context(0)
+        c.set_matmul_precision("bf16-backward")
+        m = TrainableDecisionModel(mc, c)
+        m.set_bf16_copies(copies)
+        m.set_params(params)
+        m.forward(batch, training=True, seed=5)
+        m.backward(d)
+        grads.append({n: m.grad(n) for n in m.names if m.has_grad(n)})
+        m.close()
+        c.close()
+    for n, g in grads[0].items():
+        np.testing.assert_array_equal(g, grads[1][n], err_msg=n)
+
+
+def test_split_k_rope_projection(ctx):
+    """A QKV projection past the short products' range whose 128 x 128 tiles still leave CUs idle (700 rows of 1536: 216
+    tiles, K in two): its partials are summed, rotated and measured in one pass. Against the same model on exact splits,
+    whose projection rotates in the product's epilogue: logits to 1e-5."""
+    from laya_amd.batch import synthetic_batch
+    from laya_amd.device import Context
+    from laya_amd.model import TrainableDecisionModel
+    mc = mid_config(layers=1, hidden=1536, heads=24, inter=256, head_layers=1)
+    lengths = [300, 400]
+    batch = synthetic_batch(np.random.default_rng(14), lengths, [4, 4], [0, 1], mc.encoder.vocab_size)
+    logits = []
+    for policy in ("fp32", "fp32-split3"):
+        c = Context(0)
+        c.set_matmul_precision(policy)
+        m = TrainableDecisionModel.synthetic(mc, 15, 0.03, c)
+        c.profile_begin()
+        logits.append(m.forward(batch, training=False))
+        ran = set(c.profile_end())
+        assert ({"gemm_nt_h2", "gemm_splitk_store"} <= ran) == (policy == "fp32"), ran
+        m.close()
+        c.close()
+    assert _rel(logits[0], logits[1].astype(np.float64)) < 1e-5

@@ -685,7 +685,7 @@ def test_backward_keeps_precision_for_items_with_tiny_logit_gradients(ctx):
     m.backward(dl)
     prof = ctx.profile_end()
     assert m.backward_fell_back
-    assert not any(k.endswith(("_h2w", "_h2t", "_h2")) and k.startswith(("gemm_bwd", "attention_bwd"))
+    assert not any(k.endswith(("_h2w", "_h2t", "_h2q", "_h2s", "_h2")) and k.startswith(("gemm_bwd", "attention_bwd"))
                    for k in prof), sorted(prof)
     emb = "encoder.embeddings.tok_embeddings.weight"
     exact, got = o64.grad(emb), m.grad(emb)
@@ -708,12 +708,14 @@ def test_backward_keeps_precision_for_items_with_tiny_logit_gradients(ctx):
     m.close()
 
 
-def test_adamw_step_folds_the_weights_magnitudes_exactly(ctx):
+@pytest.mark.parametrize("lengths,reads", [((150, 90, 33), False), ((512,) * 9 + (300,), True)])
+def test_adamw_step_folds_the_weights_magnitudes_exactly(ctx, lengths, reads):
     """The AdamW step folds each updated product weight's max|w| into its magnitude word, so the next forward
     measures nothing: its logits and gradients are bitwise those of a forward that measured the same weights
-    afresh (the weights written back unchanged from the host, which clears every word)."""
+    afresh (the weights written back unchanged from the host, which clears every word). Over 273 tokens most products are
+    short ones, which read no word; over 4,908 they read them."""
     from laya_amd.model import TrainableDecisionModel
-    mc, o, params, batch = _mid_case(layers=2, lengths=(150, 90, 33))
+    mc, o, params, batch = _mid_case(layers=2, lengths=lengths)
     m = TrainableDecisionModel(mc, ctx)
     m.set_params(params)
     rng = np.random.default_rng(9)
@@ -724,6 +726,7 @@ def test_adamw_step_folds_the_weights_magnitudes_exactly(ctx):
     ctx.profile_begin()
     folded = m.forward(batch, training=True, seed=3)
     prof_folded = ctx.profile_end()
+    assert not reads or any(k.startswith("gemm_nt") and k.endswith(("_h2w", "_h2t", "_h2")) for k in prof_folded)
     m.zero_gradients()
     m.backward(d)
     g_folded = {n: m.grad(n) for n in m.names if m.has_grad(n)}

@@ -235,18 +235,20 @@ def test_whole_step_from_op_entry_points_matches_the_oracle_and_the_model_driver
     om.close()
 
 
-def test_op_path_magnitude_words_change_nothing(ctx):
+@pytest.mark.parametrize("lengths,reads", [([300, 200, 129, 64, 17], False), ([512] * 9 + [300], True)])
+def test_op_path_magnitude_words_change_nothing(ctx, lengths, reads):
     """A binding that keeps the encoder operands' magnitude words (the _w entry points: producers fill them, the
     products read them instead of measuring) computes the same step as one that keeps none: each group holds
     the same largest magnitude a measuring pass would find, so the scales, the products and every gradient
-    agree bit for bit (ModernBERT-base widths, 3 encoder layers, the head and scorer, five ragged items)."""
+    agree bit for bit (ModernBERT-base widths, 3 encoder layers, the head and scorer, five ragged items, whose linears
+    are mostly short products that measure nothing, and ten of 4,908 tokens, whose products read the words)."""
     from helpers import fixture_params, mid_config, mixed_batch
     from laya_amd.device import DeviceArray
     from laya_amd.opmodel import OpBatch, OpLevelModel
     mc = mid_config(layers=3)
     o = oracle.OracleModel(mc)
     params = fixture_params(o.shapes, 31)
-    batch = mixed_batch(np.random.default_rng(32), [300, 200, 129, 64, 17], mc.encoder.vocab_size)
+    batch = mixed_batch(np.random.default_rng(32), lengths, mc.encoder.vocab_size)
     rng = np.random.default_rng(33)
     targets = np.concatenate([np.eye(k, dtype=np.float32)[rng.integers(k)] for k in batch.n_options])
     runs = []
@@ -254,10 +256,13 @@ def test_op_path_magnitude_words_change_nothing(ctx):
         om = OpLevelModel(mc, {n: params[n] for n in o.names}, ctx)
         om.carry_words = words
         ob = OpBatch(ctx, batch, targets, mc.encoder.vocab_size)
+        ctx.profile_begin()
         logits = om.forward(ob, 9, training=True)
         dl = DeviceArray(ctx, (batch.n_markers,))
         laya.softmax_ce_backward(ctx, logits, ob.targets, ob.offsets, batch.n_items, 1.0, float(batch.n_items), dl)
         om.backward(dl)
+        prof = ctx.profile_end()
+        assert not reads or any(k.startswith("gemm_nt") and k.endswith(("_h2w", "_h2t", "_h2")) for k in prof)
         runs.append((logits.numpy(), {n: om.grad(n) for n in o.names if o.has_grad(n)}))
         ob.close()
         om.close()

@@ -205,10 +205,12 @@ def test_two_piece_products_propagate_non_finite_values(ctx):
     assert rel_l2(dWc[keep], g[keep]) < 1e-6 * (rows / 2048) ** 0.5
 
 
-@pytest.mark.parametrize("rows,inn,out,with_bias", [(512, 768, 768, True), (200, 2304, 768, False)])
+@pytest.mark.parametrize("rows,inn,out,with_bias", [(512, 768, 768, True), (200, 2304, 768, False),
+                                                    (512, 784, 768, True), (200, 2320, 768, False), (200, 2320, 770, True)])
 def test_linear_in_place_residual_with_split_k(ctx, rows, inn, out, with_bias):
-    """y = x·Wᵀ + b + y with the residual being the output itself, on grids small enough (24 and 12 tiles)
-    that the product splits K and a reduce applies bias and residual."""
+    """y = x·Wᵀ + b + y with the residual being the output itself, on grids small enough (24 and 12 tiles) that K is
+    split over the chip: over the waves of the short products where K is a multiple of 32, else into partials that a
+    second pass sums with bias and residual (by fours, or one by one where the width is no multiple of 4)."""
     print(f"linear in-place residual rows={rows} in={inn} out={out}", flush=True)
     rng = np.random.default_rng(rows + inn)
     x = rng.standard_normal((rows, inn)).astype(np.float32)
@@ -217,14 +219,17 @@ def test_linear_in_place_residual_with_split_k(ctx, rows, inn, out, with_bias):
     y0 = rng.standard_normal((rows, out)).astype(np.float32)
     w, bias = param(ctx, "w", W), (param(ctx, "b", b) if with_bias else None)
     yd = dev(ctx, y0)
+    ctx.profile_begin()
     laya.linear(w, bias, dev(ctx, x), rows, yd, residual=yd)
+    assert ("gemm_splitk_store" in ctx.profile_end()) == (inn % 32 != 0)
     ref = oracle.linear(x, W, b if with_bias else None, double=True) + y0
     assert rel_l2(ref, yd.numpy()) < 1e-6
 
 
-@pytest.mark.parametrize("rows,inn,out", [(4100, 64, 96), (1500, 256, 132)])
+@pytest.mark.parametrize("rows,inn,out", [(4100, 64, 96), (1500, 256, 132), (4100, 68, 90), (1500, 250, 132)])
 def test_linear_backward_one_product(ctx, rows, inn, out):
-    """dW alone (split-K partials over a ragged last slice) and dx alone (frozen weight)."""
+    """dW alone (where a width is no multiple of 4, in split-K partials over a ragged last slice) and dx alone (frozen
+    weight)."""
     print(f"linear one-product rows={rows} in={inn} out={out}", flush=True)
     rng = np.random.default_rng(rows * 7 + inn)
     x = rng.standard_normal((rows, inn)).astype(np.float32)
@@ -234,7 +239,9 @@ def test_linear_backward_one_product(ctx, rows, inn, out):
     dx_ref = oracle.linear_backward(x, dy, W, True, dW, db, double=True)
     xd, dyd = dev(ctx, x), dev(ctx, dy)
     w = param(ctx, "w", W)
+    ctx.profile_begin()
     laya.linear_backward(w, None, xd, dyd, rows, None)
+    assert "gemm_splitk_reduce" in ctx.profile_end() or (inn % 4 == 0 and out % 4 == 0)
     assert rel_l2(dW, w.gradient.numpy()) < 1e-6
     frozen = param(ctx, "wf", W, trainable=False)
     dx_ = dev(ctx, np.zeros((rows, inn), np.float32))
@@ -392,18 +399,20 @@ def test_attention_over_many_segments(ctx):
         assert rel_l2(dref[:, sl], got[:, sl]) < 1e-5, part
 
 
-def test_operand_magnitude_ring_keeps_each_products_words():
+@pytest.mark.parametrize("inn", [64, 72])
+def test_operand_magnitude_ring_keeps_each_products_words(inn):
     """Products whose callers keep no magnitude words (the per-op entry points) measure their operands into
     the context's ring of word groups, one operand after the other. A fresh context, one attention forward
     (one measurement) to set the parity, then 130 identical linears (two measurements each) put a product's
     first measurement on every odd ring position, the wrap included; a second attention forward shifts them
     onto the even ones. Every product equals the first bit for bit: recycling the ring never clears a word
-    that a pending product still reads."""
+    that a pending product still reads. With K = 64 the linears are short products, which measure nothing, and
+    only the attention takes words; with K = 72, which those refuse, each linear takes two in one launch."""
     from laya_amd.device import Context
     c = Context(0)
     try:
         rng = np.random.default_rng(128)
-        rows, inn, out = 200, 64, 128
+        rows, out = 200, 128
         x = rng.standard_normal((rows, inn)).astype(np.float32)
         W = (0.05 * rng.standard_normal((out, inn))).astype(np.float32)
         w, xd = laya.Parameter(c, "w", W, False), dev(c, x)
@@ -416,7 +425,11 @@ def test_operand_magnitude_ring_keeps_each_products_words():
                                    dev(c, np.zeros(16, np.float32)))
             for i in range(130):
                 y = dev(c, np.zeros((rows, out), np.float32))
+                if i == 0:
+                    c.profile_begin()
                 laya.linear(w, None, xd, rows, y)
+                if i == 0:
+                    assert c.profile_end().get("absmax", {"launches": 0})["launches"] == (inn % 32 != 0)
                 got = y.numpy()
                 if first is None:
                     first = got
