@@ -59,13 +59,13 @@ def mfma_peaks(name: str):
     """(peak in algorithmic fp32 flops/s, 16-bit MFMA issues per algorithmic flop) of a matrix-core kernel.
 
     Kernels named *_x6 / *_x6w / *_x6t compute fp32 products from exact three-piece bf16 splits: six bf16
-    MFMA products per fp32 one, so their fp32-equivalent peak is the bf16 peak over six. *_h2w / *_h2t
+    MFMA products per fp32 one, so their fp32-equivalent peak is the bf16 peak over six. *_h2w / *_h2t / *_h2s
     compute them from two-piece fp16 splits of power-of-two-scaled operands: three fp16 MFMA products per
     fp32 one (fp16 and bf16 share the 2.5 PFLOP/s dense peak), peak over three; *_h2b1 / *_h2b1w / *_h2b1t
     the same with bf16-valued weights, which are one fp16 piece: two products, peak over two. *_bf16 /
-    *_bf16w run bf16 operands (one product each). The rest run the fp32 matrix cores."""
-    base = name[:-1] if name.endswith(("_x6w", "_x6t", "_bf16w", "_h2w", "_h2t", "_h2q", "_h2b1w",
-                                       "_h2b1t")) else name
+    *_bf16w / *_bf16s run bf16 operands (one product each). The rest run the fp32 matrix cores."""
+    base = name[:-1] if name.endswith(("_x6w", "_x6t", "_bf16w", "_bf16s", "_h2w", "_h2t", "_h2q", "_h2s",
+                                       "_h2b1w", "_h2b1t")) else name
     if base.endswith("_x6"):
         return PEAK_BF16_MFMA / 6, 6.0
     if base.endswith("_h2b1"):
@@ -463,9 +463,10 @@ def main():
                                    "AdamW lr 3e-5 wd 0.01, clip 1.0",
                        "global_batch": w["batch"], "seq_len": w["seq"], "parallelism": "none (1 GPU)",
                        "matmul_precision": {"fp32": "fp32-accurate products: two-piece fp16 splits of power-of-two-"
-                                                     "scaled operands on 256-wide tiles (three fp16 MFMA products "
-                                                     "each), exact three-piece bf16 splits elsewhere (six bf16 "
-                                                     "MFMA products each); fp32 accumulation",
+                                                     "scaled operands (three fp16 MFMA products each), exact "
+                                                     "three-piece bf16 splits (six bf16 MFMA products each) where "
+                                                     "an operand is not in float4s or the balanced pair of 128 x "
+                                                     "128 tiles runs; fp32 accumulation",
                                             "fp32-split3": "fp32 products from exact three-piece bf16 splits (six "
                                                            "bf16 MFMA products each, fp32 accumulation)",
                                             "fp32-mfma": "fp32 products on the fp32 MFMA",

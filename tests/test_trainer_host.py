@@ -217,3 +217,14 @@ def test_safetensors_write_replaces_the_file_whole(tmp_path):
     st = SafetensorsFile(path)
     assert list(st.entries) == ["b"]
     np.testing.assert_array_equal(st.read_float32("b"), np.ones(4, np.float32))
+
+
+@pytest.mark.parametrize("name,pieces", [("gemm_nt_h2s", 3), ("gemm_bwd_pair_h2s", 3), ("gemm_nt_h2w", 3), ("gemm_nt_h2b1t", 2),
+                                         ("gemm_nn_bf16s", 1), ("gemm_bwd_pair_bf16w", 1), ("gemm_bwd_pair_x6", 6),
+                                         ("gemm_nt", 0)])
+def test_benchmark_peaks_know_every_product_form(name, pieces):
+    """A kernel's fraction of its peak is priced by the 16-bit matrix products that one of its products takes."""
+    import bench
+    peak, issues = bench.mfma_peaks(name)
+    assert issues == pieces
+    assert peak == (bench.PEAK_BF16_MFMA / pieces if pieces else bench.PEAK_FP32_MFMA)
