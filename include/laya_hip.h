@@ -54,14 +54,17 @@ int laya_ctx_set_memory_cap(laya_ctx* ctx, size_t bytes);
 /* Precision of the matrix products launched on the context afterwards (linear layers and the model's
  * projections; the elementwise kernels stay fp32), per product class. An fp32 class (the
  * default) is computed on the 16-bit matrix cores with fp32 accumulation and fp32 results as accurate as
- * the fp32 matrix-core path (within 1e-6 relative L2 of the fp64 product on every tested shape): the
- * 256-wide kernels (the large products) split each operand, scaled by a power of two taken from its
- * largest finite magnitude, into two fp16 pieces and add three piece products per fp32 product; the
- * other kernels split each operand exactly into three bf16 pieces and add six piece products. The
- * operand-wide scale bounds the two-piece products' accuracy row by row: an output row whose operand row
- * lies 2^-k below the operand's largest keeps ≈ 2^(k-39) relative error (fp32 itself: 2^-24), so rows
- * within 2^15 of the largest are fp32-accurate, rows 2^20 below it carry ≈ 2e-6, and rows below 2^-39 of it
- * lose their precision. A caller whose rows span more selects LAYA_MATMUL_SPLIT3_* for that class; the
+ * the fp32 matrix-core path (within 1e-6 relative L2 of the fp64 product on every tested shape). Products
+ * whose k-contiguous operands allow 16-byte access split each operand, scaled by a power of two taken from its largest
+ * finite magnitude, into two fp16 pieces and add three piece products per fp32 product; the others, and the
+ * backward pairs that the 256-wide kernels refuse but a balanced plan of 128 x 128 tiles takes (5,800 to
+ * 10,800 rows of 768 -> 2304, for example), split each operand exactly into three bf16 pieces and add six
+ * piece products. The scale bounds the two-piece products' accuracy row by row: an
+ * output row whose operand row lies 2^-k below the largest that shares its scale keeps ≈ 2^(k-39) relative
+ * error (fp32 itself: 2^-24), so rows within 2^15 of the largest are fp32-accurate, rows 2^20 below it carry
+ * ≈ 2e-6, and rows below 2^-39 of it lose their precision. The scale is the operand's in the large products
+ * and a tile's in the short ones (a few thousand rows), except that short backward pairs which exact splits
+ * would compute otherwise scale each row and column by itself. A caller whose rows span more selects LAYA_MATMUL_SPLIT3_* for that class; the
  * model's backward does so by itself when the items' logit gradients span more than 2^14
  * (laya_model_backward_fallback).
  * LAYA_MATMUL_SPLIT3_* keeps a class on the three-piece splits everywhere; LAYA_MATMUL_FP32_MFMA selects

@@ -556,7 +556,6 @@ __device__ __forceinline__ void swz_col_frag(const __bf16* planes, int r0, int d
                      __builtin_bit_cast(V4, ds_read_tr(planes + pl * R * 64 + o1)));
 }
 
-// NP = 3: three-piece bf16 split products; NP = 2: two-piece fp16 products of scaled operands.
 // Short attention: workgroups of 32 rows whose four waves take a 32-row subtile of the streamed operand each, for grids
 // that would leave most of the chip idle with 128 rows to a workgroup. The waves' accumulators are summed through LDS.
 constexpr int CUT_TILE = 4 * WAVE_ROWS;
@@ -593,6 +592,8 @@ __device__ __forceinline__ unsigned store_parked(const float* red, int lane, int
     return max(amax_bits4(a), amax_bits4(b));
 }
 
+// NP = 3: three-piece bf16 split products; NP = 2: two-piece fp16 products of scaled operands. ROWS: rows to a workgroup,
+// BLOCK_ROWS or, in the short form, WAVE_ROWS.
 template <int D, bool DROP, int NP = 3, int ROWS = BLOCK_ROWS>
 __global__ __launch_bounds__(THREADS, ROWS == BLOCK_ROWS ? 2 : 1) void attn_fwd_x6_kernel(Params p) {
     static_assert(D == 64, "split-product attention is written for head_dim 64");
@@ -1571,7 +1572,7 @@ bool split_attention(const laya_ctx* ctx) { return (ctx->matmul_split | ctx->mat
 // keeps it).
 void pair_inputs(laya_ctx* ctx, const AttentionArgs& a, const float* qkv, AmaxRef r_qkv, Params& p) {
     LAYA_REQUIRE(a.rows >= 0, "attention: row count needed to measure qkv");
-    p.amax_qkv = operand_amax_ref(ctx, qkv == a.qkv ? r_qkv : AmaxRef{}, 3, qkv, a.rows, 3 * a.hidden, 3L * a.hidden);
+    p.amax_qkv = operand_amax_ref(ctx, qkv == a.qkv ? r_qkv : AmaxRef{}, qkv, a.rows, 3 * a.hidden, 3L * a.hidden);
 }
 
 }  // namespace
@@ -1655,7 +1656,7 @@ void attention_bwd(laya_ctx* ctx, const AttentionArgs& a, int rows, const float*
         p.context = const_cast<float*>(context);
         if (rot_word) {
             p.amax_qkv = rot_word;
-            p.amax_do = do_word ? do_word : operand_amax_ref(ctx, amax_do, 4, dcontext, rows, a.hidden, a.hidden);
+            p.amax_do = do_word ? do_word : operand_amax_ref(ctx, amax_do, dcontext, rows, a.hidden, a.hidden);
         } else {
             operand_amax_refs(ctx, amax_qkv, a.qkv, ar.rows, 3 * a.hidden, &p.amax_qkv, amax_do, dcontext, rows,
                               a.hidden, &p.amax_do);

@@ -351,9 +351,8 @@ void absmax_into(laya_ctx* ctx, const float* x, int rows, int cols, long ld, uns
 // aligned, device arrays of `blocks` entries) into word group word[b] of `words`; `bytes` for the profile.
 void absmax_multi(laya_ctx* ctx, const float* arena, const long* off, const int* len, const int* word, int blocks,
                   unsigned* words, double bytes);
-// An operand's magnitude word group: the caller's r (measured now if not known yet), or the context's
-// group `slot` (0 … 5), measured now.
-const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, int slot, const float* x, int rows, int cols, long ld);
+// An operand's magnitude word group: the caller's r (measured now if not known yet), or the context's next, measured now.
+const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, const float* x, int rows, int cols, long ld);
 // The same for two arrays of whole rows (ld = cols), what there is to measure in one launch.
 void operand_amax_refs(laya_ctx* ctx, AmaxRef ra, const float* a, int rows_a, int cols_a, const unsigned** word_a,
                        AmaxRef rb, const float* b, int rows_b, int cols_b, const unsigned** word_b);

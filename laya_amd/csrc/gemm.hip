@@ -1362,7 +1362,7 @@ __global__ __launch_bounds__(WT_THREADS, 1) void gemm_x6w_kernel(GemmParams p) {
 // and NaNs are left out, so the scale fits the finite values and the non-finite ones still reach the
 // products (an infinity's low piece is a NaN: outputs that an infinity reaches are non-finite, as in
 // fp32, though possibly NaN where fp32 gives an infinity).
-constexpr int AMAX_BLOCKS = 1024, AMAX_SLOTS = 6;
+constexpr int AMAX_BLOCKS = 1024;
 
 constexpr int AMAX_OPERANDS = 3;
 struct AmaxJob {
@@ -3036,8 +3036,7 @@ unsigned* operand_ring_word(laya_ctx* ctx) {
     return out;
 }
 
-const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, int slot, const float* x, int rows, int cols, long ld) {
-    LAYA_REQUIRE(slot >= 0 && slot < AMAX_SLOTS, "operand_amax_ref: no such slot");
+const unsigned* operand_amax_ref(laya_ctx* ctx, AmaxRef r, const float* x, int rows, int cols, long ld) {
     const unsigned* word = nullptr;
     operand_amaxes(ctx, {{r, x, rows, cols, ld, &word}});
     return word;

@@ -52,8 +52,8 @@ class Context:
 
     def set_matmul_precision(self, precision: str) -> None:
         """The operand precision of the matrix products launched afterwards: 'fp32' (default: fp32-accurate
-        products from exact three-piece bf16 splits on the bf16 matrix cores), 'fp32-mfma' (the fp32 matrix
-        cores), 'bf16' (every product), or one class in bf16 ('bf16-forward', 'bf16-backward',
+        products from two scaled fp16 pieces an operand, or from exact three-piece bf16 splits, on the 16-bit matrix
+        cores), 'fp32-split3' (the exact splits everywhere), 'fp32-mfma' (the fp32 matrix cores), 'bf16' (every product), or one class in bf16 ('bf16-forward', 'bf16-backward',
         'bf16-weight-grad', the other classes fp32). bf16 operands are rounded to nearest even;
         accumulation and outputs stay fp32."""
         if precision not in self.MATMUL_POLICIES:
