@@ -593,8 +593,9 @@ double traffic_of(const ShortGemm& g, long tiles_n) {
 // from the memory-side cache. Work alone does not say it: dW of 768 x 64 over 65,536 rows is twelve workgroups of 256
 // stages a wave, 460 us here and 130 with K split over the chip; 65536 x 64 -> 768 forward is 12,288 tiles of half a
 // stage a wave, 109 us here and 65 on 256-wide tiles. Fitted to 500 shapes (widths 32 … 4096, 16 … 131,072 rows, back to
-// back on one stream), where it is within 10 % for four in five. Choosing by it and by the other tiles' estimate is
-// within 1 % of the faster of the two in sum over 290 other shapes, forward, dX, dW and pair alike.
+// back on one stream), where it is within 10 % for four in five. Over 290 other shapes, forward, dX, dW and pairs,
+// choosing by it and by the other tiles' estimate is within 1 % in sum of always choosing the faster where the operands'
+// magnitudes are known, and within 3 % where they are not.
 double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, const ShortGemm& g) {
     const bool bf16 = is_bf16(ctx, layout), accumulate = ep == ShortEpilogue::Accumulate;
     const Shape s = shape_of(ctx, layout, ep, g);
@@ -607,7 +608,7 @@ double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, cons
                (each % 2) * ((accumulate ? 1.8 : 1.3) + (bf16 ? 0.6 : 1.05) * chain);
     }
     if (s.tn == 32) return 4.0 + moved + (bf16 ? 0.25 : 0.74) * ceil_div(s.tiles, 2 * cu) * chain;
-    if (s.tm == 32) return 3.6 + moved + (bf16 ? 0.8 : 1.3) * chain;
+    if (s.tm == 32) return 3.6 + moved + (bf16 ? 0.8 : 1.3) * ceil_div(s.tiles, cu) * chain;
     return 4.2 + moved + (accumulate ? 0.15 * out : 0.0) + (bf16 ? 0.95 : 1.7) * ceil_div(s.tiles, cu) * chain;
 }
 

@@ -252,11 +252,12 @@ def test_backward_pair_scaled_by_line_with_non_finite_operands(ctx):
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 @pytest.mark.parametrize("rows,fan_in,fan_out,short", [
     (13824, 768, 64, "forward"), (32768, 64, 768, "dx"), (32768, 64, 64, "forward dx"), (8192, 256, 256, "forward dx"),
-    (404, 768, 768, "forward dx dw pair"), (512, 768, 2304, "forward dx dw pair")])
+    (873, 3392, 640, "dx dw pair"), (404, 768, 768, "forward dx dw pair"), (512, 768, 2304, "forward dx dw pair")])
 def test_short_products_only_where_they_fill_the_chip(ctx, precision, rows, fan_in, fan_out, short):
     """Narrow layers over many rows: a dW of a few tiles and a long K, a forward of many tiles and a short K, and a dX of
     the same leave the short kernels, whose K is dealt to one workgroup's waves only, for the tiles that split it over
-    the chip; layers of ordinary width over few rows stay. The kernels that ran are read from the profile, the results
+    the chip, and so does a forward whose 32 x 64 tiles come in little more than one round; layers of ordinary width over
+    few rows stay. The kernels that ran are read from the profile, the results
     held to fp64 as above (dW's sums run over the rows)."""
     from laya_amd import ops
     from laya_amd.device import Context, DeviceArray
