@@ -613,7 +613,9 @@ double short_time(const laya_ctx* ctx, GemmLayout layout, ShortEpilogue ep, cons
 }
 
 // As for the forward; and eight waves where dX is few tiles of a long K, which last longest (512 x 768 -> 2304, 96
-// tiles: 27 us with eight waves, 32 with four; 800 rows, 156 tiles: 41 and 36).
+// tiles: 27 us with eight waves, 32 with four; 800 rows, 156 tiles: 41 and 36). Over 340 pairs of ordinary widths and 60 to
+// 3,000 rows the rule is within 0.6 % in sum of always taking the faster; it is furthest off where dX has 16 to 48 tiles
+// of a K under 2048 (60 x 1536 -> 1536: 17 us with eight waves, 21 with four).
 // Pairs scaled by line have at least 400 tiles: the balanced plan whose place they take needs 100 of 128 x 128 for dX.
 int pair_waves(const laya_ctx* ctx, const ShortGemm& nn, long dx_tiles, long dw_tiles, bool lines) {
     return lines || (dx_tiles + dw_tiles > ctx->cu_count && (dx_tiles >= 100 || nn.K < 2048)) ? 4 : 8;
