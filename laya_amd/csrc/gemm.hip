@@ -3322,8 +3322,9 @@ bool make_pair_plan(const laya_ctx* ctx, int n0, int out, int n1, int rows, Pair
            s.G <= FIXUP_MAX_WORKERS;
 }
 
-// The same schedule over one worker per CU, 256 x 256 tiles and 16-deep units (the wide pair); half: of bf16 products.
-bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows, bool half, PairPlan& s) {
+// The same schedule over one worker per CU, 256 x 256 tiles and 16-deep units (the wide pair); uneven: some of the workers
+// may do no dW.
+bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows, bool uneven, PairPlan& s) {
     s = PairPlan{};
     s.G = ctx->cu_count;
     s.nn_tiles = n0;
@@ -3338,10 +3339,8 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
     const long max_run = (W + s.G - 1) / s.G - (long)s.q * s.nn_units;
     // A dX tile is more than a worker's share: the workers that have one more of them do no dW, and the rest share it
     // all, while that leaves the workers at least half busy (fill): bf16 8000 x 768 -> 2304 (fill 0.74) 224 us on 128 x
-    // 128 tiles and 143 so, 4500 (0.42) 111 and 117. Not for fp32 products: most of these shapes run as exact
-    // three-piece splits (make_pair_plan), which keep rows of dY far below its largest that two pieces under one scale
-    // would round away, and three-piece units take twice as long here.
-    if (half && need_min < 0 && s.nn_units > 0 && 2 * W >= (long)s.G * (s.q + 1) * s.nn_units) {
+    // 128 tiles and 143 so, 4500 (0.42) 111 and 117; fp32 5400 x 1024 -> 5248 510 and 453.
+    if (uneven && need_min < 0 && s.nn_units > 0 && 2 * W >= (long)s.G * (s.q + 1) * s.nn_units) {
         const long dW = (long)n1 * s.tn_units, workers = s.G - s.r;
         s.rest = true;
         return (dW + workers - 1) / workers < s.tn_units && W < (1L << 30) && s.G <= FIXUP_MAX_WORKERS;
@@ -3351,8 +3350,7 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
 }
 
 // The wide pair for split products: dX without residual, dX's K a multiple of 16, dY k-contiguous in
-// float4s. Returns false (nothing launched) when the wide plan does not apply, or is an uneven one where `uneven` is
-// not set: launches of their own are faster for a bf16 dX of few tiles (3232 x 1152 -> 768: 56 us and 62).
+// float4s. Returns false (nothing launched) when the wide plan does not apply (uneven: that of make_pair_plan_wide).
 // amax_dx (optional): dX's magnitude word group, folded in by the two-piece kernel (*folded set), else
 // left to the caller.
 bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, int in, int out, bool half,
@@ -3367,7 +3365,7 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
     tn.tiles_n = (in + WT - 1) / WT;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;
     PairPlan s{};
-    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, half, s) || (s.rest && !uneven)) return false;
+    if (!make_pair_plan_wide(ctx, n0, out, n1, rows, uneven, s)) return false;
     s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * WT * WT));
     const bool pair = !half && (ctx->matmul_pair & 6) == 6;
     if (pair) {
@@ -3432,28 +3430,36 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
                              const __bf16* x16, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx,
                              bool* folded) {
     if (rows == 0) return;
-    bool uneven = true;  // whether the wide pair may leave dW to some of its workers
+    bool uneven = false;  // whether the wide pair may leave dW to some of its workers
     {
         ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
         const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
         nn.amax = amax_dx;
         // Against the wide pair's longest worker and its fixup, us fitted to 60 shapes each (a unit is a 256 x 256 x 16
-        // product), or dX and dW in launches of their own, less what the second saves by following the first.
+        // product), or dX and dW in launches of their own, less what the second saves by following the first, and at least
+        // what 128 x 128 tiles take for their work (5400 x 1024 -> 5248: fp32 510 us, bf16 351).
         const bool bf16 = (ctx->matmul_bf16 & 6) == 6;
         const int wt_in = (in + WT - 1) / WT, t_in = (in + BN - 1) / BN;
-        PairPlan s{};
-        const bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
-                                                               (out + WT - 1) / WT * wt_in, rows, bf16, s);
         PairPlan balanced{};  // of 128 x 128 tiles
         const bool planned =
             make_pair_plan(ctx, (rows + BM - 1) / BM * t_in, out, (out + BM - 1) / BM * t_in, rows, balanced);
-        double other = (bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
-                       (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16);
+        // Not in place of that plan's exact three-piece splits, which keep rows of dY far below its largest that two
+        // pieces under one scale would round away, and not as three-piece products, whose units take twice as long.
+        uneven = bf16 || (!planned && !(ctx->matmul_bf16 & 6) && (ctx->matmul_pair & ctx->matmul_split & 6) == 6);
+        PairPlan s{};
+        bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
+                                                         (out + WT - 1) / WT * wt_in, rows, uneven, s);
+        const double work = (double)rows * in * out;
+        double other = std::max((bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
+                                    (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16),
+                                2.0 * (bf16 ? 6.3e-9 : 9.5e-9) * work);
         if (wide && s.rest) {
-            const double rest =
-                25.0 + 0.75 * std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
-            uneven = planned || rest < other;
-            if (uneven) other = rest;
+            // Nor where launches of their own are faster (bf16 3232 x 1152 -> 768 56 us and 62, fp32 5400 x 768 -> 2304 193
+            // and 214), unless the balanced plan, slower by far, would come next.
+            const double units = std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
+            const double rest = bf16 ? 25.0 + 0.75 * units : 32.0 + 1.3 * units;
+            uneven = wide = planned || rest < other;
+            if (wide) other = rest;
         } else if (wide) {
             other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
         } else if (planned && !bf16) {

@@ -135,12 +135,13 @@ def test_short_attention(ctx, lengths, window, p_drop):
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 @pytest.mark.parametrize("rows,fan_in,fan_out,bf16_kernel", [
     (2500, 3072, 768, "gemm_bwd_pair_bf16w"), (6000, 768, 2304, "gemm_bwd_pair_bf16w"),
-    (8003, 768, 2304, "gemm_bwd_pair_bf16w"), (5300, 768, 2304, ""), (6001, 768, 768, ""), (3232, 1152, 768, "gemm_nn_bf16")])
+    (8003, 768, 2304, "gemm_bwd_pair_bf16w"), (5300, 768, 2304, ""), (6001, 768, 768, ""), (3232, 1152, 768, "gemm_nn_bf16"),
+    (5500, 1024, 5248, "gemm_bwd_pair_bf16w")])
 def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in, fan_out, bf16_kernel):
     """Pairs whose dX tile is more than a worker's share of the wide plan. In bf16 the workers with one more dX tile do no
     dW where that pays (the shapes that name the wide kernel: half of the workers busy, and either the balanced plan of
-    128 x 128 tiles would be next or launches of their own are not faster); in fp32 none does. Against fp64 on the same
-    operands, 1e-6 relative L2 widened by the square root of K over 768 for dW, whose sums run over the rows."""
+    128 x 128 tiles would be next or launches of their own are not faster); in fp32 only where exact splits would not be
+    next and launches of their own are slower (the last shape). Against fp64 on the same operands, 1e-6 relative L2 widened by the square root of K over 768 for dW, whose sums run over the rows."""
     from laya_amd import ops
     from laya_amd.device import Context, DeviceArray
     c = ctx if precision == "fp32" else Context(0)
@@ -154,7 +155,7 @@ def test_backward_pair_of_few_input_gradient_tiles(ctx, precision, rows, fan_in,
     c.profile_begin()
     ops.linear_backward(Wp, None, DeviceArray.from_numpy(c, x), DeviceArray.from_numpy(c, dy), rows, dx)
     ran = set(c.profile_end())
-    assert not any(k.endswith("_h2w") for k in ran)
+    assert ("gemm_bwd_pair_h2w" in ran) == (precision == "fp32" and fan_out == 5248), ran
     assert precision == "fp32" or not bf16_kernel or bf16_kernel in ran, ran
     assert _rel(dx.numpy(), low(dy) @ low(W)) < 1e-6
     assert _rel(Wp.gradient_buffer().numpy(), low(dy).T @ low(x)) < 1e-6 * np.sqrt(rows / 768)
