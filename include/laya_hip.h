@@ -57,8 +57,8 @@ int laya_ctx_set_memory_cap(laya_ctx* ctx, size_t bytes);
  * the fp32 matrix-core path (within 1e-6 relative L2 of the fp64 product on every tested shape). Products
  * whose k-contiguous operands allow 16-byte access split each operand, scaled by a power of two taken from its largest
  * finite magnitude, into two fp16 pieces and add three piece products per fp32 product; the others, and the
- * backward pairs that the 256-wide kernels refuse but a balanced plan of 128 x 128 tiles takes (5,800 to
- * 10,800 rows of 768 -> 2304, for example), split each operand exactly into three bf16 pieces and add six
+ * backward pairs that the 256-wide kernels' balanced plan refuses and one of 128 x 128 tiles takes (5,800
+ * to 10,800 rows of 768 -> 2304, for example), split each operand exactly into three bf16 pieces and add six
  * piece products. The scale bounds the two-piece products' accuracy row by row: an
  * output row whose operand row lies 2^-k below the largest that shares its scale keeps ≈ 2^(k-39) relative
  * error (fp32 itself: 2^-24), so rows within 2^15 of the largest are fp32-accurate, rows 2^20 below it carry

@@ -3351,10 +3351,11 @@ bool make_pair_plan_wide(const laya_ctx* ctx, int n0, int out, int n1, int rows,
 
 // The wide pair for split products: dX without residual, dX's K a multiple of 16, dY k-contiguous in
 // float4s. Returns false (nothing launched) when the wide plan does not apply (uneven: that of make_pair_plan_wide).
+// exact: three-piece splits whatever the policy.
 // amax_dx (optional): dX's magnitude word group, folded in by the two-piece kernel (*folded set), else
 // left to the caller.
 bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, int in, int out, bool half,
-                        bool uneven, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx, bool* folded) {
+                        bool uneven, bool exact, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx, bool* folded) {
     const bool bh = half && nn.B16 && tn.B16;  // W and x from their bf16 copies
     if (out % BKQ != 0 || !operand_fast(nn.A, nn.lda, nn.vec_a, true, nn.M, nn.K)) return false;
     const long lim = 1L << 31;  // buffer offsets of dY, W and x
@@ -3367,7 +3368,7 @@ bool backward_pair_wide(laya_ctx* ctx, GemmParams nn, GemmParams tn, int rows, i
     PairPlan s{};
     if (!make_pair_plan_wide(ctx, n0, out, n1, rows, uneven, s)) return false;
     s.partial = static_cast<float*>(ctx->workspace(0, sizeof(float) * (size_t)s.G * 2 * WT * WT));
-    const bool pair = !half && (ctx->matmul_pair & 6) == 6;
+    const bool pair = !half && !exact && (ctx->matmul_pair & 6) == 6;
     if (pair) {
         operand_amaxes(ctx, {{amax_dy, nn.A, rows, out, nn.lda, &nn.amax_a},
                              {amax_W, nn.B, out, in, nn.ldb, &nn.amax_b},
@@ -3430,7 +3431,8 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
                              const __bf16* x16, AmaxRef amax_dy, AmaxRef amax_W, AmaxRef amax_x, unsigned* amax_dx,
                              bool* folded) {
     if (rows == 0) return;
-    bool uneven = false;  // whether the wide pair may leave dW to some of its workers
+    // Whether the wide pair may leave dW to some of its workers, and whether it takes exact splits then.
+    bool uneven = false, exact = false;
     {
         ShortGemm nn = short_params(rows, in, out, dy, out, W, in, dx, in, nullptr, dx_residual, in);
         const ShortGemm tn = short_params(out, in, rows, dy, out, x, in, dW, in, nullptr, nullptr, 0);
@@ -3443,9 +3445,8 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         PairPlan balanced{};  // of 128 x 128 tiles
         const bool planned =
             make_pair_plan(ctx, (rows + BM - 1) / BM * t_in, out, (out + BM - 1) / BM * t_in, rows, balanced);
-        // Not in place of that plan's exact three-piece splits, which keep rows of dY far below its largest that two
-        // pieces under one scale would round away, and not as three-piece products, whose units take twice as long.
-        uneven = bf16 || (!planned && !(ctx->matmul_bf16 & 6) && (ctx->matmul_pair & ctx->matmul_split & 6) == 6);
+        const bool two_piece = !(ctx->matmul_bf16 & 6) && (ctx->matmul_pair & ctx->matmul_split & 6) == 6;
+        uneven = bf16 || two_piece;
         PairPlan s{};
         bool wide = out % BKQ == 0 && make_pair_plan_wide(ctx, (rows + WT - 1) / WT * wt_in, out,
                                                          (out + WT - 1) / WT * wt_in, rows, uneven, s);
@@ -3453,20 +3454,26 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
         double other = std::max((bf16 ? 6.0 : 4.0) + 0.92 * tiles_time(ctx, rows, in, out, bf16) +
                                     (bf16 ? 0.75 : 0.9) * tiles_time(ctx, out, in, rows, bf16),
                                 2.0 * (bf16 ? 6.3e-9 : 9.5e-9) * work);
+        const double balanced_us = 25.0 + 3.1 * balanced.W / balanced.G;
         if (wide && s.rest) {
-            // Nor where launches of their own are faster (bf16 3232 x 1152 -> 768 56 us and 62, fp32 5400 x 768 -> 2304 193
-            // and 214), unless the balanced plan, slower by far, would come next.
+            // Not where launches of their own are faster (bf16 3232 x 1152 -> 768 56 us and 62, fp32 5400 x 768 -> 2304 193
+            // and 214). Where the balanced plan would come next, which bf16 products are slower with by far, fp32 ones
+            // stay exact three-piece splits, as there: they keep rows of dY far below its largest that two pieces under
+            // one scale would round away (8000 x 1024 -> 3072 594 us on that plan and 455 here, 10000 x 768 -> 2304 428
+            // and 335, 5400 x 1024 -> 1024 150 and 160).
             const double units = std::max((s.q + 1.0) * s.nn_units, (double)s.tn_tiles * s.tn_units / (s.G - s.r));
-            const double rest = bf16 ? 25.0 + 0.75 * units : 32.0 + 1.3 * units;
-            uneven = wide = planned || rest < other;
+            const double rest = bf16 ? 25.0 + 0.75 * units : planned ? 28.0 + 2.08 * units : 32.0 + 1.3 * units;
+            if (planned && !bf16) other = balanced_us;
+            uneven = wide = (planned && bf16) || rest < other;
+            exact = wide && planned && !bf16;
             if (wide) other = rest;
         } else if (wide) {
             other = 40.0 + (bf16 ? 1.1 : 1.6) * s.W / s.G;
         } else if (planned && !bf16) {
-            other = 55.0 + 2.15 * balanced.W / balanced.G;
+            other = balanced_us;
         }
         other += measuring_time(bf16, (double)rows * out + (double)out * in + (double)rows * in);
-        const bool lines = !bf16 && !wide && planned;  // exact three-piece splits would follow
+        const bool lines = !bf16 && planned && (!wide || exact);  // exact three-piece splits would follow
         if (short_pair_pays(ctx, nn, tn, lines, other)) {
             short_gemm_pair(ctx, nn, tn, lines);
             *folded = amax_dx != nullptr;
@@ -3487,7 +3494,8 @@ void gemm_backward_pair_body(laya_ctx* ctx, int rows, int in, int out, const flo
     const bool half = (ctx->matmul_bf16 & 6) == 6 && gemm_fits_h(nn, true, false) && gemm_fits_h(tn, false, false);
     tn.mode = ACCUMULATE;
     if ((split || half) &&
-        backward_pair_wide(ctx, nn, tn, rows, in, out, half, uneven, amax_dy, amax_W, amax_x, amax_dx, folded))
+        backward_pair_wide(ctx, nn, tn, rows, in, out, half, uneven, exact, amax_dy, amax_W, amax_x, amax_dx,
+                           folded))
         return;
     tn.mode = STORE;
     const int n0 = nn.tiles_m * nn.tiles_n, n1 = tn.tiles_m * tn.tiles_n;

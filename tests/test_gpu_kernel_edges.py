@@ -193,7 +193,7 @@ def test_uneven_wide_pair_with_a_residual(ctx):
 
 
 @pytest.mark.parametrize("rows,fan_in,fan_out,kernel", [
-    (12345, 768, 700, "x6"), (8003, 768, 2304, "x6"), (5600, 768, 768, "x6"), (2500, 3072, 768, "h2s"),
+    (12345, 768, 700, "x6"), (8003, 768, 2304, "x6w"), (7001, 1020, 1024, "x6w"), (5600, 768, 768, "x6"), (2500, 3072, 768, "h2s"),
     (1400, 3072, 768, "h2s"), (1403, 3076, 800, "h2s"), (1600, 2624, 1024, "h2s")])
 def test_backward_pairs_keep_lines_far_below_the_largest(ctx, rows, fan_in, fan_out, kernel):
     """fp32 backward pairs on exact three-piece splits, or on two pieces scaled by row and column: rows and columns of dY,
