@@ -3010,8 +3010,8 @@ double tiles_time(const laya_ctx* ctx, int M, int N, int K, bool bf16, bool one_
 }
 
 // What to count of measuring an fp32 product's operands, 3.3 us and 0.14 per MB where their magnitudes are not known: half
-// of it whether they are known or not, so that a caller who keeps them gets the same bits as one who does not. Over 3,300
-// products that costs the one 1 % and the other 3 % of the time that choosing by what is known would give.
+// of it whether they are known or not, so that a caller who keeps them gets the same bits as one who does not. Over 3,400
+// products that costs each of them 1 % of the time that choosing by what is known would give.
 double measuring_time(bool bf16, double elements) { return bf16 ? 0.0 : 0.5 * (3.3 + 0.14 * 4e-6 * elements); }
 
 // A product's time with that: A is M x K and B N x K, however they are stored.

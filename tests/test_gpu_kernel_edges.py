@@ -298,6 +298,31 @@ def test_short_products_only_where_they_fill_the_chip(ctx, precision, rows, fan_
         c.close()
 
 
+@pytest.mark.parametrize("rows,fan_in,fan_out,backward", [(3200, 1152, 768, False), (4500, 1152, 768, True)])
+def test_fp32_products_of_even_estimates_run_short(ctx, rows, fan_in, fan_out, backward):
+    """Where the estimates do not tell which tiles are faster, the short kernels take the product: each of a workgroup's
+    waves sums its share of K in 32-bit accumulators of its own, a quarter of a sequential sum's terms or fewer. With
+    independent rounding errors of at most 2^-24 of a partial sum, a sum of K / 16 matrix instructions over four waves
+    stays below sqrt(K / 64) x 2^-24 of its norm (2.5e-7 for K = 1152, 2.1e-7 for 768), and the two pieces of an operand
+    leave out less than 2^-22 of each value, independently: together below 5e-7."""
+    from laya_amd import ops
+    from laya_amd.device import DeviceArray
+    r = np.random.default_rng(rows)
+    W = (0.02 * r.standard_normal((fan_out, fan_in))).astype(np.float32)
+    a = r.standard_normal((rows, fan_out if backward else fan_in)).astype(np.float32)
+    frozen, ad = ops.Parameter(ctx, "F", W, False), DeviceArray.from_numpy(ctx, a)
+    out = DeviceArray(ctx, (rows, fan_in if backward else fan_out))
+    ctx.profile_begin()
+    if backward:
+        x = DeviceArray.from_numpy(ctx, np.zeros((rows, fan_in), np.float32))
+        ops.linear_backward(frozen, None, x, ad, rows, out)
+    else:
+        ops.linear(frozen, None, ad, rows, out)
+    assert any(k.startswith("gemm_nn" if backward else "gemm_nt") and k.endswith("_h2s") for k in ctx.profile_end())
+    W64 = W.astype(np.float64)
+    assert _rel(out.numpy(), a.astype(np.float64) @ (W64 if backward else W64.T)) < 5e-7
+
+
 @pytest.mark.parametrize("policy", ["fp32", "fp32-split3", "fp32-mfma"])
 @pytest.mark.parametrize("head_dim,lengths,window", [(64, [300, 65], -1), (64, [700, 129], 64), (32, [200, 33], 8)])
 def test_attention_backward_in_place(head_dim, lengths, window, policy):
